@@ -528,8 +528,8 @@ vs_status vs_scene_bvh_export(const vs_scene *s, const uint32_t **nodes, uint32_
                               const float **leaf_tris, uint32_t *num_leaf_tris) {
     if (!s || !nodes || !num_nodes || !leaf_tris || !num_leaf_tris) return VS_ERROR_INVALID_ARGUMENT;
     if (!s->host_bvh) return fail(s->ctx, VS_ERROR_STATE, "bvh not built");
-    *nodes = reinterpret_cast<const uint32_t *>(s->bvh.nodes.data());
-    *num_nodes = uint32_t(s->bvh.nodes.size());
+    *nodes = reinterpret_cast<const uint32_t *>(s->bvh.export_nodes.data());
+    *num_nodes = uint32_t(s->bvh.export_nodes.size());
     *leaf_tris = reinterpret_cast<const float *>(s->bvh.tris.data());
     *num_leaf_tris = uint32_t(s->bvh.tris.size());
     return VS_OK;

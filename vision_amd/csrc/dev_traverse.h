@@ -19,10 +19,15 @@ namespace vs {
 namespace dev {
 
 struct RayPre {
-    f3 o, d;
+    f3 o;
     float tmin;
     f3 idir;
-    uint32_t oct;
+    // visiting order: the halves, quarters and eighths of the slots that the
+    // ray meets first
+    uint32_t first4, first2, first1;
+    // byte selectors of the planes the ray enters by: slots 0 and 1 of a low
+    // and a high plane word, into the low bytes of the two halves
+    uint32_t near_x, near_y, near_z;
     int kx, ky, kz;
     float Sx, Sy, Sz;
 };
@@ -37,10 +42,14 @@ __device__ __forceinline__ float safe_rcp(float d) {
 __device__ __forceinline__ RayPre make_ray_pre(f3 o, f3 d, float tmin) {
     RayPre r;
     r.o = o;
-    r.d = d;
     r.tmin = tmin;
     r.idir = mk3(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-    r.oct = (d.x < 0.f ? 1u : 0u) | (d.y < 0.f ? 2u : 0u) | (d.z < 0.f ? 4u : 0u);
+    r.first1 = d.x < 0.f ? 0xAAu : 0x55u;
+    r.first2 = d.y < 0.f ? 0xCCu : 0x33u;
+    r.first4 = d.z < 0.f ? 0xF0u : 0x0Fu;
+    r.near_x = r.idir.x >= 0.f ? 0x0C010C00u : 0x0C050C04u;
+    r.near_y = r.idir.y >= 0.f ? 0x0C010C00u : 0x0C050C04u;
+    r.near_z = r.idir.z >= 0.f ? 0x0C010C00u : 0x0C050C04u;
     float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     int kz = ax > ay ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
     int kx = kz + 1 == 3 ? 0 : kz + 1;
@@ -60,9 +69,10 @@ __device__ __forceinline__ RayPre make_ray_pre(f3 o, f3 d, float tmin) {
     return r;
 }
 
-// watertight ray/triangle test; returns false on a miss
-__device__ __forceinline__ bool intersect_triangle(const RayPre &r, f3 v0, f3 v1, f3 v2,
-                                                   float &t, float &b1, float &b2) {
+// watertight ray/triangle test; returns false on a miss.  The barycentrics
+// of a hit are V / det and W / det: only the closest hit's are divided.
+__device__ __forceinline__ bool intersect_triangle(const RayPre &r, f3 v0, f3 v1, f3 v2, float &t, float &V, float &W,
+                                                   float &det) {
 #pragma clang fp contract(off)
     f3 A = v0 - r.o, B = v1 - r.o, C = v2 - r.o;
     float Akz = sel3(A, r.kz), Bkz = sel3(B, r.kz), Ckz = sel3(C, r.kz);
@@ -73,9 +83,9 @@ __device__ __forceinline__ bool intersect_triangle(const RayPre &r, f3 v0, f3 v1
     float Cx = sel3(C, r.kx) - r.Sx * Ckz;
     float Cy = sel3(C, r.ky) - r.Sy * Ckz;
     float U = Cx * By - Cy * Bx;
-    float V = Ax * Cy - Ay * Cx;
-    float W = Bx * Ay - By * Ax;
-    if (U == 0.f || V == 0.f || W == 0.f) {
+    V = Ax * Cy - Ay * Cx;
+    W = Bx * Ay - By * Ax;
+    if (fminf(fminf(fabsf(U), fabsf(V)), fabsf(W)) == 0.f) {
         double CxBy = double(Cx) * double(By), CyBx = double(Cy) * double(Bx);
         U = float(CxBy - CyBx);
         double AxCy = double(Ax) * double(Cy), AyCx = double(Ay) * double(Cx);
@@ -83,14 +93,13 @@ __device__ __forceinline__ bool intersect_triangle(const RayPre &r, f3 v0, f3 v1
         double BxAy = double(Bx) * double(Ay), ByAx = double(By) * double(Ax);
         W = float(BxAy - ByAx);
     }
-    if ((U < 0.f || V < 0.f || W < 0.f) && (U > 0.f || V > 0.f || W > 0.f)) return false;
-    float det = U + V + W;
-    if (det == 0.f) return false;
+    det = U + V + W;
+    // both signs among the three: outside
+    const bool out = (fminf(fminf(U, V), W) < 0.f) & (fmaxf(fmaxf(U, V), W) > 0.f);
+    if (out | (det == 0.f)) return false;
     float Az = r.Sz * Akz, Bz = r.Sz * Bkz, Cz = r.Sz * Ckz;
     float T = U * Az + V * Bz + W * Cz;
     t = T / det;
-    b1 = V / det;
-    b2 = W / det;
     return true;
 }
 
@@ -100,65 +109,100 @@ struct TraceHit {
     float b1, b2;
 };
 
-__device__ __forceinline__ uint32_t permute_oct(uint32_t m, uint32_t oct) {
-    if (oct & 1u) m = ((m & 0x55u) << 1) | ((m & 0xAAu) >> 1);
-    if (oct & 2u) m = ((m & 0x33u) << 2) | ((m & 0xCCu) >> 2);
-    if (oct & 4u) m = ((m & 0x0Fu) << 4) | ((m & 0xF0u) >> 4);
-    return m;
+// byte i of the result: byte sel[i] of lo (0..3) or hi (4..7), or zero (0x0C)
+__device__ __forceinline__ uint32_t pick_bytes(uint32_t hi, uint32_t lo, uint32_t sel) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_perm(hi, lo, sel);
+#else
+    uint32_t r = 0;
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t b = (sel >> (8 * i)) & 0xFFu;
+        if (b < 8u) r |= (((b < 4u ? lo : hi) >> (8u * (b & 3u))) & 0xFFu) << (8 * i);
+    }
+    return r;
+#endif
 }
 
-__device__ __forceinline__ float qbyte(uint32_t lo_word, uint32_t hi_word, int s) {
-    uint32_t w = s < 4 ? lo_word : hi_word;
-    return float((w >> ((s & 3) * 8)) & 0xFFu);
+// the low (0) or high (1) half of a word whose halves hold bytes, read as a
+// half-precision value: byte * 2^-24
+__device__ __forceinline__ float byte_half(uint32_t w, int hi) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return float(__builtin_bit_cast(_Float16, uint16_t(hi ? w >> 16 : w)));
+#else
+    return float(hi ? w >> 16 : w & 0xFFFFu) * 0x1p-24f;
+#endif
 }
 
-// intersect the 8 child boxes of node `idx`; outputs the internal-child hit
-// mask in visiting order and the leaf-triangle mask relative to tri_base
-__device__ __forceinline__ void process_node(const uint4 *__restrict__ nodes, uint32_t idx, const RayPre &r,
-                                             float tmax, uint32_t &cbase, uint32_t &chits, uint32_t &cimask,
-                                             uint32_t &tbase, uint32_t &tmask, uint32_t &nfetch) {
+// Intersect the 8 child boxes of node `idx` (layout in bvh.h).  Out: the
+// internal children hit, by slot, with child_base and imask; the triangles of
+// the leaves hit as bits of the node's leaf mask, with that mask and the
+// node's first triangle.
+// Bound by VALU issue and, close behind, by the texture addresser, which
+// takes a 16-byte load's 64 lanes some 20 cycles whether active or not.  So
+// the node stays at five loads, and a child costs 3 byte picks (two planes
+// each; they choose near and far on the way), 6 mixed-precision FMAs on the
+// picked bytes as half denormals, 4 min / max, and a subtract whose sign bit
+// is shifted into the miss mask: 15 instructions for 21 with a conversion a
+// plane, selects and a compare.
+__device__ __forceinline__ void process_node(const uint4 *__restrict__ nodes, uint32_t idx, const RayPre &r, float tmax,
+                                             uint32_t &cbase, uint32_t &chits, uint32_t &cimask, uint32_t &tbase,
+                                             uint32_t &tleaf, uint32_t &tmask, uint32_t &nfetch) {
     const uint4 *np = nodes + size_t(idx) * 5;
-    uint4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3], n4 = np[4];
+    const uint4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3], n4 = np[4];
     ++nfetch;
-    float sx = __uint_as_float((n0.w & 0xFFu) << 23) * r.idir.x;
-    float sy = __uint_as_float(((n0.w >> 8) & 0xFFu) << 23) * r.idir.y;
-    float sz = __uint_as_float(((n0.w >> 16) & 0xFFu) << 23) * r.idir.z;
-    float ax = (__uint_as_float(n0.x) - r.o.x) * r.idir.x;
-    float ay = (__uint_as_float(n0.y) - r.o.y) * r.idir.y;
-    float az = (__uint_as_float(n0.z) - r.o.z) * r.idir.z;
-    bool px = r.idir.x >= 0.f, py = r.idir.y >= 0.f, pz = r.idir.z >= 0.f;
-    // per axis the quantised planes the ray enters and leaves by: the low
-    // ones first where its direction is positive (chosen once per node, not
-    // per child)
-    const uint32_t nx0 = px ? n2.x : n3.z, nx1 = px ? n2.y : n3.w, fx0 = px ? n3.z : n2.x, fx1 = px ? n3.w : n2.y;
-    const uint32_t ny0 = py ? n2.z : n4.x, ny1 = py ? n2.w : n4.y, fy0 = py ? n4.x : n2.z, fy1 = py ? n4.y : n2.w;
-    const uint32_t nz0 = pz ? n3.x : n4.z, nz1 = pz ? n3.y : n4.w, fz0 = pz ? n4.z : n3.x, fz1 = pz ? n4.w : n3.y;
-    uint32_t imask = n0.w >> 24;
-    uint32_t hitmask = 0;
+    const float sx = __uint_as_float(n0.w << 16) * r.idir.x;
+    const float sy = __uint_as_float(n0.w & 0xFFFF0000u) * r.idir.y;
+    const float sz = __uint_as_float(n1.w & 0xFFFF0000u) * r.idir.z;
+    const float ax = (__uint_as_float(n0.x) - r.o.x) * r.idir.x;
+    const float ay = (__uint_as_float(n0.y) - r.o.y) * r.idir.y;
+    const float az = (__uint_as_float(n0.z) - r.o.z) * r.idir.z;
+    uint32_t miss = 0;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        float nx = fmaf(qbyte(nx0, nx1, s), sx, ax), fx = fmaf(qbyte(fx0, fx1, s), sx, ax);
-        float ny = fmaf(qbyte(ny0, ny1, s), sy, ay), fy = fmaf(qbyte(fy0, fy1, s), sy, ay);
-        float nz = fmaf(qbyte(nz0, nz1, s), sz, az), fz = fmaf(qbyte(fz0, fz1, s), sz, az);
-        float tn = fmaxf(fmaxf(nx, ny), fmaxf(nz, r.tmin));
-        float tf = fminf(fminf(fx, fy), fminf(fz, tmax));
-        hitmask |= (tn <= tf ? 1u : 0u) << s;
-    }
-    uint32_t leafhits = hitmask & ~imask;
-    uint32_t tm = 0;
+    for (int k = 3; k >= 0; --k) {
+        // slots 2 k and 2 k + 1
+        const uint32_t up = (k & 1) ? 0x00020002u : 0u;
+        const uint32_t lx = k < 2 ? n2.x : n2.y, ly = k < 2 ? n2.z : n2.w, lz = k < 2 ? n3.x : n3.y;
+        const uint32_t hx = k < 2 ? n3.z : n3.w, hy = k < 2 ? n4.x : n4.y, hz = k < 2 ? n4.z : n4.w;
+        const uint32_t nx = pick_bytes(hx, lx, r.near_x + up), fx = pick_bytes(lx, hx, r.near_x + up);
+        const uint32_t ny = pick_bytes(hy, ly, r.near_y + up), fy = pick_bytes(ly, hy, r.near_y + up);
+        const uint32_t nz = pick_bytes(hz, lz, r.near_z + up), fz = pick_bytes(lz, hz, r.near_z + up);
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        uint32_t meta = ((s < 4 ? n1.z : n1.w) >> ((s & 3) * 8)) & 0xFFu;
-        uint32_t cnt = meta >> 5, off = meta & 31u;
-        uint32_t bits = ((1u << cnt) - 1u) << off;
-        tm |= (leafhits >> s) & 1u ? bits : 0u;
+        for (int b = 1; b >= 0; --b) {
+            const float tn = fmaxf(fmaxf(fmaf(byte_half(nx, b), sx, ax), fmaf(byte_half(ny, b), sy, ay)),
+                                   fmaxf(fmaf(byte_half(nz, b), sz, az), r.tmin));
+            const float tf = fminf(fminf(fmaf(byte_half(fx, b), sx, ax), fmaf(byte_half(fy, b), sy, ay)),
+                                   fminf(fmaf(byte_half(fz, b), sz, az), tmax));
+            miss = (miss << 1) | (__float_as_uint(tf - tn) >> 31);
+        }
     }
-    tmask = tm;
+    const uint32_t hits = ~miss & 0xFFu;
+    cimask = n1.z >> 24;
+    chits = hits & cimask;
+    // slot s to bits 3 s .. 3 s + 2; slots that are no leaves are not in the leaf mask
+    uint32_t m = hits;
+    m = (m | (m << 8)) & 0x00F00Fu;
+    m = (m | (m << 4)) & 0x0C30C3u;
+    m = (m | (m << 2)) & 0x249249u;
+    tleaf = n1.z;// its high byte lies above every triangle's bit
+    tmask = (m | (m << 1) | (m << 2)) & n1.z;
     tbase = n1.y;
     cbase = n1.x;
-    cimask = imask;
-    chits = permute_oct(hitmask & imask, r.oct);
 }
+
+// the slot of `hits` that the ray meets first: its mask bit
+__device__ __forceinline__ uint32_t first_slot(uint32_t hits, const RayPre &r) {
+    uint32_t m = hits & r.first4;
+    m = m ? m : hits;
+    uint32_t n = m & r.first2;
+    n = n ? n : m;
+    m = n & r.first1;
+    return m ? m : n;
+}
+
+// boxes are culled against a slightly later t than the closest hit's: the
+// slab test and the triangle test round differently, and of triangles in one
+// plane that overlap the lower id has to be found
+__device__ __forceinline__ float box_limit(float t) { return fmaf(fabsf(t), 0x1p-20f, t); }
 
 template <bool ANY>
 __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, float tmin, float tmax,
@@ -169,26 +213,31 @@ __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, fl
     TraceHit h;
     h.t = tmax;
     h.tri = kInvalid;
-    h.b1 = h.b2 = 0.f;
+    float hV = 0.f, hW = 0.f, hdet = 1.f;
     uint32_t sp = 0;
-    uint32_t gbase, ghits, gimask, tbase, tmask;
-    process_node(nodes, 0, r, tmax, gbase, ghits, gimask, tbase, tmask, nfetch);
+    uint32_t gbase, ghits, gimask, tbase, tleaf, tmask;
+    process_node(nodes, 0, r, box_limit(tmax), gbase, ghits, gimask, tbase, tleaf, tmask, nfetch);
     while (true) {
         while (tmask) {
-            uint32_t j = __builtin_ctz(tmask);
-            tmask &= tmask - 1u;
-            const float4 *tp = ltri + size_t(tbase + j) * 3;
+            const uint32_t bit = tmask & (0u - tmask);
+            tmask ^= bit;
+            const float4 *tp = ltri + size_t(tbase + uint32_t(__popc(tleaf & (bit - 1u)))) * 3;
             float4 a = tp[0], b = tp[1], c = tp[2];
             ++tfetch;
-            float t, b1, b2;
-            if (intersect_triangle(r, mk3(a.x, a.y, a.z), mk3(b.x, b.y, b.z), mk3(c.x, c.y, c.z), t, b1, b2)) {
-                uint32_t id = __float_as_uint(a.w);
-                if (t > tmin && t < tmax && (t < h.t || (t == h.t && id < h.tri))) {
+            float t, V, W, det;
+            if (intersect_triangle(r, mk3(a.x, a.y, a.z), mk3(b.x, b.y, b.z), mk3(c.x, c.y, c.z), t, V, W, det)) {
+                const uint32_t id = __float_as_uint(a.w);
+                if ((t > tmin) & (t < tmax) & ((t < h.t) | ((t == h.t) & (id < h.tri)))) {
                     h.t = t;
                     h.tri = id;
-                    h.b1 = b1;
-                    h.b2 = b2;
-                    if (ANY) return h;
+                    hV = V;
+                    hW = W;
+                    hdet = det;
+                    if (ANY) {
+                        h.b1 = V / det;
+                        h.b2 = W / det;
+                        return h;
+                    }
                 }
             }
         }
@@ -200,12 +249,11 @@ __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, fl
             ghits = e.y & 0xFFu;
             gimask = e.y >> 8;
         }
-        uint32_t i = __builtin_ctz(ghits);
-        ghits &= ghits - 1u;
-        uint32_t slot = i ^ r.oct;
-        uint32_t child = gbase + __popc(gimask & ((1u << slot) - 1u));
+        const uint32_t bit = first_slot(ghits, r);
+        ghits ^= bit;
+        const uint32_t child = gbase + uint32_t(__popc(gimask & (bit - 1u)));
         uint32_t nb, nh, ni;
-        process_node(nodes, child, r, ANY ? tmax : h.t, nb, nh, ni, tbase, tmask, nfetch);
+        process_node(nodes, child, r, box_limit(ANY ? tmax : h.t), nb, nh, ni, tbase, tleaf, tmask, nfetch);
         if (nh) {
             if (ghits) {
                 if (sp < sc.stack_size) stack[sp * stride] = make_uint2(gbase, ghits | (gimask << 8));
@@ -217,6 +265,9 @@ __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, fl
             gimask = ni;
         }
     }
+    // zero on a miss (0 / 1)
+    h.b1 = hV / hdet;
+    h.b2 = hW / hdet;
     return h;
 }
 
