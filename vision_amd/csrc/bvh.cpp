@@ -152,46 +152,17 @@ void set_byte(uint32_t *w, int word0, int slot, uint32_t v) {
     word = (word & ~(0xFFu << sh)) | ((v & 0xFFu) << sh);
 }
 
-// the smallest float of 16 significant bits (sign, exponent, 7 bits of
-// fraction) that is not below v > 0
-uint32_t step_bits(double v) {
-    float f = float(v);
-    if (double(f) < v) f = std::nextafter(f, FLT_MAX);
-    return (fbits(f) + 0xFFFFu) >> 16;
-}
-
-// Frame and planes of the traversal's node: origin a step below the padded
-// box, steps for the span of the box and one more on each side, each child's
-// planes a step outside its box
-void wide_node(const Box &nb, const Box *child, uint32_t slots, Bvh8Node &node) {
-    uint32_t step16[3];
-    for (int a = 0; a < 3; ++a) {
-        const double lo = comp(nb.lo, a), hi = comp(nb.hi, a);
-        const double mag = std::max(std::fabs(lo), std::fabs(hi));
-        const double margin = mag * std::ldexp(1.0, -18) + 1e-30;
-        // 255 steps: the span, one on each side, one for each rounding below
-        step16[a] = step_bits(std::ldexp(std::max((hi - lo + 2.0 * margin) / 250.0, 1e-30), 24));
-        const uint32_t sb = step16[a] << 16;
-        float sf;
-        std::memcpy(&sf, &sb, 4);
-        const double step = std::ldexp(double(sf), -24);
-        float pf = float(lo - margin - step);
-        if (double(pf) > lo - margin - step) pf = std::nextafter(pf, -FLT_MAX);
-        node.w[a] = fbits(pf);
-        for (int s = 0; s < 8; ++s) {
-            uint32_t ql = 255, qh = 0;// empty slot: inverted, never hit
-            if (slots >> s & 1u) {
-                const double l = std::floor((double(comp(child[s].lo, a)) - double(pf)) / step) - 1.0;
-                const double h = std::ceil((double(comp(child[s].hi, a)) - double(pf)) / step) + 1.0;
-                ql = uint32_t(std::min(std::max(l, 0.0), 255.0));
-                qh = uint32_t(std::min(std::max(h, 0.0), 255.0));
-            }
-            set_byte(node.w, 8 + 2 * a, s, ql);
-            set_byte(node.w, 14 + 2 * a, s, qh);
-        }
-    }
-    node.w[3] = step16[0] | step16[1] << 16;
-    node.w[7] = step16[2] << 16;
+// the traversal's node (bvh.h): the same frame and planes, steps and the
+// leaves' triangles in the form it takes them
+Bvh8Node traversal_node(const Bvh8ExportNode &n, uint32_t leaf_mask) {
+    Bvh8Node r{};
+    std::copy(n.w, n.w + 20, r.w);
+    uint32_t step[3];
+    for (int a = 0; a < 3; ++a) step[a] = std::min(((n.w[3] >> (8 * a)) & 0xFFu) + 24u, 254u) << 7;
+    r.w[3] = step[0] | step[1] << 16;
+    r.w[6] = leaf_mask | (n.w[3] & 0xFF000000u);
+    r.w[7] = step[2] << 16;
+    return r;
 }
 
 }// namespace
@@ -324,14 +295,11 @@ Bvh8 build_bvh8(const std::vector<f3> &P, const std::vector<u3> &tris) {
         std::vector<int> by_slot(8, -1);
         for (size_t c = 0; c < ch.size(); ++c) by_slot[size_t(slot_of[c])] = int(c);
         uint32_t tri_off = 0;
-        Box slot_box[8];
-        uint32_t slots = 0, leaf_mask = 0;
+        uint32_t leaf_mask = 0;
         for (int s = 0; s < 8; ++s) {
             int c = by_slot[size_t(s)];
             if (c < 0) continue;
             const Node2 &cn = N2[ch[size_t(c)]];
-            slots |= 1u << s;
-            slot_box[s] = cn.box;
             for (int a = 0; a < 3; ++a) {
                 double lo = comp(cn.box.lo, a), hi = comp(cn.box.hi, a);
                 double ql = std::floor((lo - origin[a]) / step[a]) - 1.0;
@@ -369,12 +337,7 @@ Bvh8 build_bvh8(const std::vector<f3> &P, const std::vector<u3> &tris) {
         if (tri_off > 24) throw std::runtime_error("bvh: leaf triangle budget exceeded");
         w[3] |= imask << 24;
         out.export_nodes[pend.node8] = node;
-        Bvh8Node wide{};
-        wide_node(nb, slot_box, slots, wide);
-        wide.w[4] = child_base;
-        wide.w[5] = tri_base;
-        wide.w[6] = leaf_mask | imask << 24;
-        out.nodes.push_back(wide);// breadth first: node8 counts up by one
+        out.nodes.push_back(traversal_node(node, leaf_mask));// breadth first: node8 counts up by one
     }
     out.sah_cost = sah;
     return out;

@@ -13,9 +13,9 @@
 namespace vs {
 
 // The node the traversal reads (5 x 16 B):
-//  w[0..2]  frame origin p (float bits)
+//  w[0..2]  origin p (float bits)
 //  w[3]     steps of x (low half) and y (high half), w[7] high half: z; a half
-//           is the upper 16 bits of the float 2^24 * step
+//           is the upper 16 bits of the float 2^24 * step, step = 2^e
 //  w[4]     child_base: index of the first internal child node
 //  w[5]     tri_base:   index of the first leaf triangle of this node
 //  w[6]     leaf mask: bit 3 s + k set when slot s is a leaf with more than k
@@ -26,8 +26,7 @@ namespace vs {
 // Two bytes put into the low bytes of a word's halves are two half-precision
 // values q * 2^-24 (denormals, exact), which the mixed-precision FMA of the
 // slab test takes as operands (traversal, process_node): the 2^24 is in the
-// steps.  Planes are at least one step (1/250 of the frame) outside the
-// child's box, more than the rounding of the slab tests, so no hit is culled.
+// steps.
 //
 // Slot s holds the child whose centre lies most toward the octant direction
 // ((s&1)?+x:-x, (s&2)?+y:-y, (s&4)?+z:-z); a ray whose direction-sign bits are

@@ -199,11 +199,6 @@ __device__ __forceinline__ uint32_t first_slot(uint32_t hits, const RayPre &r) {
     return m ? m : n;
 }
 
-// boxes are culled against a slightly later t than the closest hit's: the
-// slab test and the triangle test round differently, and of triangles in one
-// plane that overlap the lower id has to be found
-__device__ __forceinline__ float box_limit(float t) { return fmaf(fabsf(t), 0x1p-20f, t); }
-
 template <bool ANY>
 __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, float tmin, float tmax,
                                              uint2 *stack, uint32_t stride, uint32_t &nfetch, uint32_t &tfetch) {
@@ -216,7 +211,7 @@ __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, fl
     float hV = 0.f, hW = 0.f, hdet = 1.f;
     uint32_t sp = 0;
     uint32_t gbase, ghits, gimask, tbase, tleaf, tmask;
-    process_node(nodes, 0, r, box_limit(tmax), gbase, ghits, gimask, tbase, tleaf, tmask, nfetch);
+    process_node(nodes, 0, r, tmax, gbase, ghits, gimask, tbase, tleaf, tmask, nfetch);
     while (true) {
         while (tmask) {
             const uint32_t bit = tmask & (0u - tmask);
@@ -253,7 +248,7 @@ __device__ __forceinline__ TraceHit traverse(const SceneView &sc, f3 o, f3 d, fl
         ghits ^= bit;
         const uint32_t child = gbase + uint32_t(__popc(gimask & (bit - 1u)));
         uint32_t nb, nh, ni;
-        process_node(nodes, child, r, box_limit(ANY ? tmax : h.t), nb, nh, ni, tbase, tleaf, tmask, nfetch);
+        process_node(nodes, child, r, ANY ? tmax : h.t, nb, nh, ni, tbase, tleaf, tmask, nfetch);
         if (nh) {
             if (ghits) {
                 if (sp < sc.stack_size) stack[sp * stride] = make_uint2(gbase, ghits | (gimask << 8));
