@@ -224,8 +224,9 @@ vs_status vs_trace_closest_noalloc(vs_scene *scene, const vs_ray *rays, uint32_t
 vs_status vs_scene_bsdf(vs_scene *scene, uint32_t mat, uint32_t n, const float *wo, const float *wi,
                         const float *lambda, int32_t sample, uint32_t frame, float *wi_out, float *f, float *pdf);
 
-/* Kernel form of vs_render.  MEGAKERNEL: one thread per pixel runs whole
- * paths (fused or per-frame launches).  WAVEFRONT: the bounce loop split into
+/* Kernel form of vs_render.  MEGAKERNEL: a thread runs whole paths (fused or
+ * per-frame launches; a fused job of several frames may run its samples in
+ * threads of their own, or as wavefront, where that is faster).  WAVEFRONT: the bounce loop split into
  * closest-hit / shade / any-hit kernels over queues of live paths held in
  * HBM, `chunk_frames` frames of all pixels per chunk, traversal blocks of
  * `trace_block` (64, 128 or 256) threads.  Both give the same film.  No

@@ -1,0 +1,59 @@
+"""The megakernel form's fused jobs of several frames on the MI355X: whichever
+way vs_render runs them (a lane a sample for the diffuse family, as wavefront
+for every material, one lane a pixel where counters or adaptive sampling need
+it), the film and the output buffer equal the frame-by-frame launches' bit for
+bit, also continued from an earlier frame, at odd sizes and without
+accumulation."""
+import numpy as np
+import pytest
+
+from vision_amd import scenegen
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(kind, folder):
+    if kind == "diffuse":
+        return scenegen.cornell_box(64, 64, max_depth=5)
+    return scenegen.procedural_scene(folder, n_instances=4, level=2, width=64, height=64, max_depth=6, hdri=(64, 32),
+                                     spectrum="srgb")
+
+
+@pytest.mark.parametrize("kind", ["diffuse", "materials"])
+@pytest.mark.parametrize("size,spp,first", [((1, 1), 3, 0), ((8, 8), 2, 0), ((9, 17), 3, 1), ((65, 63), 7, 2)])
+@pytest.mark.parametrize("spectral", [0, 3, 4])
+def test_fused_equals_frame_by_frame(gpu_ctx, tmp_path, kind, size, spp, first, spectral):
+    sc = gpu_ctx.load_text(_scene(kind, tmp_path), str(tmp_path))
+    sc.build_accel()
+    sc.set_resolution(*size)
+    if spectral:
+        sc.set_spectrum(True, spectral)
+    films = []
+    for fused in (False, True):
+        sc.reset_film()
+        if first:
+            sc.render(first, fused=False)
+        sc.render(spp, fused=fused)
+        assert sc.info()["frame_index"] == first + spp
+        films.append((sc.film(0), sc.film(1)))
+    for a, b in zip(*films):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    sc.set_counting(True)
+    sc.reset_film()
+    sc.render(first + spp)
+    assert sc.stats()["rays"] > 0
+    assert np.array_equal(sc.film(0).view(np.uint32), films[0][0].view(np.uint32))
+    sc.close()
+
+
+def test_last_frame_without_accumulation(gpu_ctx):
+    s = scenegen.cornell_box(40, 24, max_depth=4)
+    s["camera"]["param"]["radiance_collector"]["param"]["accumulation"] = 0
+    sc = gpu_ctx.load_text(s)
+    sc.build_accel()
+    sc.render(3, fused=False)
+    a = sc.film(0)
+    sc.reset_film()
+    sc.render(3)
+    assert np.array_equal(a.view(np.uint32), sc.film(0).view(np.uint32))
+    sc.close()

@@ -54,6 +54,7 @@ struct DevBuf {
         hipError_t e = hipMalloc(&ptr, n);
         if (e != hipSuccess) {
             ptr = nullptr;
+            (void)hipGetLastError();// the next launch does not report it again
             throw DeviceError(std::string("hipMalloc failed: ") + hipGetErrorString(e));
         }
         bytes = n;
@@ -128,6 +129,7 @@ struct vs_scene {
     bool diffuse_only{false};// only diffuse / Oren-Nayar / black materials
     DevBuf fis_lut, fis_cond, fis_cond_func, fis_marg, fis_marg_func;
     DevBuf film_rt, film_out, film_pic, counters;
+    DevBuf samples;// radiance of single camera samples (sample megakernel)
     DevBuf scratch_rays, scratch_hits;
     // wavefront form: per-path state, queues, append counters
     uint32_t kernel_mode{VS_KERNEL_MEGAKERNEL};
@@ -225,6 +227,9 @@ inline void require_built(vs_scene *s) {
 // live-path queue until it empties, then the chunk folds into the film.
 // Synchronises `st` once per bounce (the live count).  Returns launches;
 // adds per-stage times to *ts when it and the three events are given.
+// wavefront_reserve: path state for `paths` paths; false (and nothing held)
+// when the device has no room.
+bool wavefront_reserve(WavefrontBuffers &wb, size_t paths);
 uint32_t wavefront_render(const vs::SceneView &view, const vs::CameraView &cam, const vs::RenderView &rv0,
                           bool rgb, bool diffuse_only, float4 *rt, float4 *out, uint32_t frame_index, uint32_t spp, uint32_t chunk,
                           uint32_t trace_block, WavefrontBuffers &wb, hipStream_t st, unsigned long long *ctr,

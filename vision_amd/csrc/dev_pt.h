@@ -678,5 +678,25 @@ __device__ __forceinline__ void render_column(const SceneView &sc, const CameraV
     }
 }
 
+// The radiance of one camera sample, film weight applied: the path that
+// render_column runs for this pixel and frame
+template <int NS, bool RGB, int MS>
+__device__ __forceinline__ f3 render_sample(const SceneView &sc, const CameraView &cam, const RenderView &rv,
+                                            uint32_t px, uint32_t py, uint32_t frame, uint2 *stack, uint32_t stride) {
+    uint32_t dn = 0, dt = 0;
+    PathState<NS> ps;
+    path_begin<NS, RGB>(cam, rv, px, py, frame, ps);
+    while (ps.alive) {
+        TraceHit h = traverse<false>(sc, ps.o, ps.d, 0.f, 3.402823466e38f, stack, stride, dn, dt);
+        ShadowRay sr;
+        path_shade<NS, RGB, MS>(sc, rv, ps, h, sr);
+        if (sr.valid) {
+            TraceHit sh = traverse<true>(sc, sr.o, sr.d, 0.f, 1.f - kShadowEpsilon, stack, stride, dn, dt);
+            if (sh.tri == kInvalid) ps.L += sr.c;
+        }
+    }
+    return ps.L * ps.fw;
+}
+
 }// namespace dev
 }// namespace vs

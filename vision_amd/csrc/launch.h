@@ -17,6 +17,12 @@ hipError_t launch_bsdf(const SceneView &sc, uint32_t spectrum_dim, uint32_t mat,
 // (the kernel is compiled without the other material families)
 hipError_t launch_pt(const SceneView &sc, const CameraView &cam, const RenderView &rv, float4 *rt, float4 *out,
                      unsigned long long *counters, bool diffuse_only, hipStream_t stream);
+// The frames rv.frame_start .. + rv.spp (at most 65535) of the same job, a
+// lane a sample, each one's radiance into L[frame * pixels + pixel]; the film
+// then takes them in frame order (wf_accumulate).  Diffuse-family scenes,
+// without adaptive sampling and counters.
+hipError_t launch_pt_samples(const SceneView &sc, const CameraView &cam, const RenderView &rv, float4 *L,
+                             hipStream_t stream);
 // the saved picture: tone map (again) + optional sRGB gamma over the output buffer (film.hip)
 hipError_t launch_final_picture(const float4 *in, float4 *out, uint32_t n, uint32_t tone_mapper, bool gamma,
                                 hipStream_t stream);
