@@ -69,14 +69,27 @@ struct NrcQuery {
     uint32_t pad;
 };
 
+// Workspace of the network's kernels, for `rows` rows at a time: the features
+// of a row (16 words of two bf16, level-major) and, for the backward pass, their
+// gradients (32 floats) and the weight gradients and loss of
+// nrc_backward_blocks() blocks.  Lists longer than that run in chunks.
+constexpr int kNrcPartial = kNrcMlpParams + 1;
+struct NrcScratch {
+    uint32_t *feat;
+    float *dx, *partial;
+    uint32_t rows;
+};
+
 // ---- kernels (nrc.hip) ----
 // parity and utility entry points over n positions / samples
-hipError_t nrc_forward(const NrcView &v, const float *pos, uint32_t n, float *out, hipStream_t s);
+hipError_t nrc_forward(const NrcView &v, const float *pos, uint32_t n, float *out, const NrcScratch &sc,
+                       hipStream_t s);
+uint32_t nrc_backward_blocks();
 // forward + backward over samples [offset, offset + batch) of the
 // min(*count, capacity) present: gradients of their mean loss accumulate
 // into v.mlp_g / v.grid_g, the mean loss into *loss (all must start at zero)
 hipError_t nrc_backward(const NrcView &v, const NrcSample *samples, const uint32_t *count, uint32_t capacity,
-                        uint32_t offset, uint32_t batch, float *loss, uint32_t blocks, hipStream_t s);
+                        uint32_t offset, uint32_t batch, float *loss, const NrcScratch &sc, hipStream_t s);
 // Adam step over all parameters with bias corrections c1 = 1 / (1 - 0.9^t),
 // c2 = 1 / (1 - 0.99^t); clears the gradients and refreshes the fp16 /
 // bf16 copies
@@ -85,7 +98,7 @@ hipError_t nrc_adam(const NrcView &v, float lr, float c1, float c2, hipStream_t 
 hipError_t nrc_sync_copies(const NrcView &v, hipStream_t s);
 // queries: out radiance added into L[slot] += beta * max(y, 0)
 hipError_t nrc_infer(const NrcView &v, const NrcQuery *q, const uint32_t *count, uint32_t capacity, float4 *L,
-                     hipStream_t s);
+                     const NrcScratch &sc, hipStream_t s);
 
 // rendering with the cache (sRGB mode): one thread per (pixel, sample) of
 // a frame; paths stop at bounce `term` and append a query, radiance so far

@@ -8,6 +8,7 @@
 #include "nrc.h"
 
 #include <algorithm>
+#include <cstddef>
 
 namespace vs {
 
@@ -18,6 +19,14 @@ namespace {
 constexpr int kBlock = 256;// 4 waves
 constexpr uint32_t kTrainStream = 1u << 30;
 
+// The rows of a launch: the min(*count, cap) (or cap) present from `offset` on,
+// the offset taken modulo that number, at most `batch`
+__device__ __forceinline__ uint32_t nrc_rows(const uint32_t *count, uint32_t cap, uint32_t &offset, uint32_t batch) {
+    const uint32_t total = count ? min(*count, cap) : cap;
+    if (total) offset %= total;
+    return min(total - (total ? offset : 0u), batch);
+}
+
 // per-wave LDS of the forward-only kernels: one 16-row tile at a time
 // (features, two hidden buffers used in turn, outputs), so that twelve
 // waves per CU fit beside the block's weights
@@ -27,8 +36,8 @@ struct NrcFwdLds {
     float y[16 * 4];
 };
 
-// forward of one row tile (the arithmetic of nrc_forward_tile with the
-// hidden buffers reused: H3 overwrites H1 once layer 2 has read it)
+// forward of one row tile, the hidden buffers reused: H3 overwrites H1 once
+// layer 2 has read it
 __device__ __forceinline__ void fwd_tile(const NrcWeightsLds &w, NrcFwdLds &s, int lane) {
     nrc_fwd_tile<kNrcIn, kNrcHidden>(s.x, kXs, w.w1t, kXs, s.h[0], lane);
     __builtin_amdgcn_wave_barrier();
@@ -36,47 +45,85 @@ __device__ __forceinline__ void fwd_tile(const NrcWeightsLds &w, NrcFwdLds &s, i
     __builtin_amdgcn_wave_barrier();
     nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[1], kHs, w.w3t, kHs, s.h[0], lane);
     __builtin_amdgcn_wave_barrier();
-    if (lane < 48) {
-        int row = lane / 3, c = lane % 3;
-        float acc = 0.f;
-        for (int k = 0; k < kNrcHidden; ++k) acc += bf2f(s.h[0][row * kHs + k]) * w.w4[k * kNrcOut + c];
-        s.y[row * 4 + c] = acc;
-    }
+    nrc_out_tile(s.h[0], w.w4, s.y, lane);
     __builtin_amdgcn_wave_barrier();
 }
 
-// INFER: rows are queries (count on the device), their radiance goes into
-// L; otherwise rows are n positions and outputs go to out[n][3]
-template <bool INFER>
-__global__ void __launch_bounds__(kBlock) nrc_forward_kernel(NrcView v, const float *__restrict__ pos, uint32_t n_pos,
-                                                             const NrcQuery *__restrict__ q,
-                                                             const uint32_t *__restrict__ count, uint32_t cap,
-                                                             float *__restrict__ out, float4 *__restrict__ L) {
-    __shared__ NrcWeightsLds w;
-    __shared__ NrcFwdLds ws[kBlock / 64];
-    nrc_load_weights(v, w, threadIdx.x, kBlock);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    NrcFwdLds &s = ws[wave];
-    const uint32_t n = INFER ? min(*count, cap) : n_pos;
-    for (uint32_t base = (blockIdx.x * (kBlock / 64) + wave) * 64u; base < n; base += gridDim.x * kBlock) {
-        const uint32_t row = base + lane;
-        const bool valid = row < n;
+// Features of the rows [first, first + span) of a list of positions, `stride`
+// floats apart, `count` (on the device, when given; at most cap) or cap of them
+// in all: feat[level][row - first], two bf16 a word.
+// A wave takes Q x 64 rows and goes through the levels in the outer loop, so
+// that the whole GPU gathers from about one level's table (2 MB of 32) at a
+// time: it stays in every XCD's L2, and the coarse ones in L1.  With a row's
+// levels one after the other the gathers missed L2 half the time and ran at
+// the Infinity Cache's bandwidth (7.5 TB/s): a full-HD frame's queries took
+// 1.92 ms, now 1.43 ms (1.08 of them here).
+template <int Q>
+__global__ void __launch_bounds__(kBlock) nrc_encode_kernel(NrcView v, const float *__restrict__ pos, uint32_t stride,
+                                                            const uint32_t *__restrict__ count, uint32_t cap,
+                                                            uint32_t offset, uint32_t batch, uint32_t first,
+                                                            uint32_t span, uint32_t *__restrict__ feat) {
+    const uint32_t n = nrc_rows(count, cap, offset, batch);
+    const uint32_t end = min(n, first + span);
+    const uint32_t base = first + (blockIdx.x * kBlock + (threadIdx.x & ~63u)) * Q + (threadIdx.x & 63u);
+    if (first + blockIdx.x * kBlock * Q >= end) return;
+    float u[Q][3];
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
         float p[3] = {0.f, 0.f, 0.f};
-        if (valid) {
-            const float *src = INFER ? q[row].p : pos + 3 * size_t(row);
+        const uint32_t row = base + 64u * j;
+        if (row < end) {
+            const float *src = pos + size_t(offset + row) * stride;
             p[0] = src[0];
             p[1] = src[1];
             p[2] = src[2];
         }
-        uint16_t x[kNrcIn];
-        nrc_encode(v, p, x);
+        nrc_unit(v, p, u[j]);
+    }
+    const uint32_t *table = reinterpret_cast<const uint32_t *>(v.grid_f16);
+#pragma unroll 1
+    for (int l = 0; l < kNrcLevels; ++l, table += kNrcTable) {
+        const bool dense = (v.dense_mask >> l) & 1u;
+#pragma unroll
+        for (int j = 0; j < Q; ++j) {
+            const uint32_t row = base + 64u * j;
+            if (row >= end) continue;
+            float a0, a1;
+            if (dense) nrc_level<true>(table, v.res[l], u[j], a0, a1);
+            else nrc_level<false>(table, v.res[l], u[j], a0, a1);
+            feat[size_t(l) * span + (row - first)] = uint32_t(f2bf(a0)) | uint32_t(f2bf(a1)) << 16;
+        }
+    }
+}
+
+// The network over encoded rows.  INFER: rows are queries (count on the
+// device), their radiance goes into L; otherwise outputs go to out[row][3]
+template <bool INFER>
+__global__ void __launch_bounds__(kBlock) nrc_forward_kernel(NrcView v, const uint32_t *__restrict__ feat,
+                                                             const NrcQuery *__restrict__ q,
+                                                             const uint32_t *__restrict__ count, uint32_t cap,
+                                                             uint32_t first, uint32_t span, float *__restrict__ out,
+                                                             float4 *__restrict__ L) {
+    __shared__ NrcWeightsLds w;
+    __shared__ NrcFwdLds ws[kBlock / 64];
+    const uint32_t n = INFER ? min(*count, cap) : cap;
+    const uint32_t end = min(n, first + span);
+    if (first + blockIdx.x * kBlock >= end) return;
+    nrc_load_weights<kBlock>(v, w, nullptr, threadIdx.x);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    NrcFwdLds &s = ws[wave];
+    for (uint32_t base = first + (blockIdx.x * (kBlock / 64) + wave) * 64u; base < end; base += gridDim.x * kBlock) {
+        const uint32_t row = base + lane;
+        const bool valid = row < end;
+        uint32_t x[kNrcLevels];
+#pragma unroll
+        for (int l = 0; l < kNrcLevels; ++l) x[l] = valid ? feat[size_t(l) * span + (row - first)] : 0u;
         for (int rt = 0; rt < 4; ++rt) {
             if ((lane >> 4) == rt) {
 #pragma unroll
-                for (int k = 0; k < kNrcIn; k += 4)
-                    *reinterpret_cast<bf16x4 *>(s.x + (lane & 15) * kXs + k) =
-                        bf16x4{short(x[k]), short(x[k + 1]), short(x[k + 2]), short(x[k + 3])};
+                for (int l = 0; l < kNrcLevels; l += 2)
+                    *reinterpret_cast<uint2 *>(s.x + (lane & 15) * kXs + 2 * l) = make_uint2(x[l], x[l + 1]);
             }
             __builtin_amdgcn_wave_barrier();
             fwd_tile(w, s, lane);
@@ -101,85 +148,190 @@ __global__ void __launch_bounds__(kBlock) nrc_forward_kernel(NrcView v, const fl
     }
 }
 
-// forward + backward over the training samples; one block per CU loops
-// over chunks of 64 samples per wave, weight gradients gather in LDS and
-// reach global memory once per block
-__global__ void __launch_bounds__(kBlock) nrc_backward_kernel(NrcView v, const NrcSample *__restrict__ samples,
-                                                              const uint32_t *__restrict__ count, uint32_t cap,
-                                                              uint32_t offset, uint32_t batch,
-                                                              float *__restrict__ loss) {
+// The network forward and backward over encoded training samples, rows
+// [first, first + span) of the step's; the features' gradients go to
+// dx[row - first][32].  A wave takes 16 rows at a time.  The weight gradients
+// stay in MFMA accumulators over all rows of a wave and meet in LDS once (added
+// to LDS tile by tile they were 2300 LDS atomics a wave), and a layer's
+// gradient overwrites its activations, so that eight waves fit beside the
+// weights.  Blocks hand their sums to nrc_reduce_kernel: 256 blocks' atomics on
+// the same 10432 parameters took 100 of 135 us.
+// A step's gradients for 65536 samples took 1030 us in one kernel of four waves
+// a CU that also gathered and scattered a row a lane; now 430 us: encoding
+// 29, this and the reduction 135, scatter 220 to 265.
+constexpr int kBackWaves = 8;
+constexpr int kBackBlock = 64 * kBackWaves;
+struct NrcBackWaveLds {
+    uint16_t x[16 * kXs];   // features of the tile
+    uint16_t h[3][16 * kHs];// H1..H3 (post-ReLU), then the gradients there
+    float y[16 * 4];        // outputs, then dL/dy
+};
+struct NrcGradLds {
+    float w1[kNrcIn * kNrcHidden];
+    float w2[kNrcHidden * kNrcHidden];
+    float w3[kNrcHidden * kNrcHidden];
+    float w4[kNrcHidden * kNrcOut];
+    float loss;
+};
+static_assert(offsetof(NrcGradLds, loss) == sizeof(float) * kNrcMlpParams && kNrcW1 == 0, "layers in parameter order");
+
+__global__ void __launch_bounds__(kBackBlock) nrc_backward_kernel(NrcView v, const NrcSample *__restrict__ samples,
+                                                                  const uint32_t *__restrict__ feat,
+                                                                  const uint32_t *__restrict__ count, uint32_t cap,
+                                                                  uint32_t offset, uint32_t batch, uint32_t first,
+                                                                  uint32_t span, float *__restrict__ dx,
+                                                                  float *__restrict__ partial) {
     __shared__ NrcWeightsLds w;
-    __shared__ NrcGradLds gl;
-    __shared__ NrcWaveLds ws[kBlock / 64];
-    nrc_load_weights(v, w, threadIdx.x, kBlock);
-    for (int i = threadIdx.x; i < kNrcIn * kNrcHidden; i += kBlock) gl.w1[i] = 0.f;
-    for (int i = threadIdx.x; i < kNrcHidden * kNrcHidden; i += kBlock) {
-        gl.w2[i] = 0.f;
-        gl.w3[i] = 0.f;
+    __shared__ NrcBackWeightsLds wb;
+    __shared__ union {
+        NrcBackWaveLds wave[kBackWaves];
+        NrcGradLds grad;// once the waves are through
+    } sh;
+    const uint32_t n = nrc_rows(count, cap, offset, batch);
+    const uint32_t end = min(n, first + span);
+    partial += size_t(blockIdx.x) * kNrcPartial;
+    if (first + blockIdx.x * uint32_t(kBackWaves * 16) >= end) {
+        for (int i = threadIdx.x; i < kNrcPartial; i += kBackBlock) partial[i] = 0.f;
+        return;
     }
-    for (int i = threadIdx.x; i < kNrcHidden * kNrcOut; i += kBlock) gl.w4[i] = 0.f;
+    samples += offset;
+    nrc_load_weights<kBackBlock>(v, w, &wb, threadIdx.x);
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    NrcWaveLds &s = ws[wave];
-    // this step's samples: [offset, offset + batch) of the min(*count, cap)
-    // present, the offset taken modulo that count
-    const uint32_t total = min(*count, cap);
-    if (total) offset %= total;
-    const uint32_t n = min(total - offset, batch);
-    samples += offset;
-    const float inv = n ? 1.f / (3.f * float(n)) : 0.f;
+    NrcBackWaveLds &s = sh.wave[wave];
+    const float inv = 1.f / (3.f * float(n));
     float loss_acc = 0.f;
-    for (uint32_t base = (blockIdx.x * (kBlock / 64) + wave) * 64u; base < n; base += gridDim.x * kBlock) {
-        const uint32_t row = base + lane;
-        const bool valid = row < n;
-        float p[3] = {0.f, 0.f, 0.f}, t[3] = {0.f, 0.f, 0.f};
-        if (valid) {
-            const NrcSample &sm = samples[row];
-            p[0] = sm.p[0];
-            p[1] = sm.p[1];
-            p[2] = sm.p[2];
-            t[0] = sm.t[0];
-            t[1] = sm.t[1];
-            t[2] = sm.t[2];
-        }
-        uint16_t x[kNrcIn];
-        nrc_encode(v, p, x);
+    f32x4 g1[kNrcIn / 16][4] = {}, g2[4][4] = {}, g3[4][4] = {};
+    float g4[3] = {0.f, 0.f, 0.f};
+    const float w4r[3] = {w.w4[lane * 3], w.w4[lane * 3 + 1], w.w4[lane * 3 + 2]};
+    const uint32_t step = gridDim.x * uint32_t(kBackWaves * 16);
+    for (uint32_t base = first + (blockIdx.x * kBackWaves + wave) * 16u; base < end; base += step) {
+        // lane: row of 16 x a quarter of the levels
+        const int i = lane & 15;
+        const bool valid = base + i < end;
+        const uint32_t present = uint32_t(__ballot(valid)) & 0xFFFFu;
 #pragma unroll
-        for (int k = 0; k < kNrcIn; k += 4)
-            *reinterpret_cast<bf16x4 *>(s.x + lane * kXs + k) = bf16x4{short(x[k]), short(x[k + 1]),
-                                                                         short(x[k + 2]), short(x[k + 3])};
+        for (int k = 0; k < kNrcLevels / 4; ++k) {
+            const int l = (lane >> 4) * (kNrcLevels / 4) + k;
+            const uint32_t f = valid ? feat[size_t(l) * span + (base + i - first)] : 0u;
+            *reinterpret_cast<uint32_t *>(s.x + i * kXs + 2 * l) = f;
+        }
         __builtin_amdgcn_wave_barrier();
-        for (int rt = 0; rt < 4; ++rt) {
-            nrc_forward_tile(w, s, rt, lane);
-            if ((lane >> 4) == rt) {
-                const int i = lane & 15;
+        nrc_fwd_tile<kNrcIn, kNrcHidden>(s.x, kXs, w.w1t, kXs, s.h[0], lane);
+        __builtin_amdgcn_wave_barrier();
+        nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[0], kHs, w.w2t, kHs, s.h[1], lane);
+        __builtin_amdgcn_wave_barrier();
+        nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[1], kHs, w.w3t, kHs, s.h[2], lane);
+        __builtin_amdgcn_wave_barrier();
+        nrc_out_tile(s.h[2], w.w4, s.y, lane);
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 16) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    float y = s.y[i * 4 + c];
-                    float d = y - t[c];
-                    float den = y * y + 0.01f;
-                    loss_acc += valid ? d * d / den * inv : 0.f;
-                    s.y[i * 4 + c] = valid ? 2.f * d / den * inv : 0.f;
-                }
+            for (int c = 0; c < 3; ++c) {
+                const float t = valid ? samples[base + i].t[c] : 0.f;
+                const float y = s.y[i * 4 + c];
+                const float d = y - t;
+                const float den = y * y + 0.01f;
+                loss_acc += valid ? d * d / den * inv : 0.f;
+                s.y[i * 4 + c] = valid ? 2.f * d / den * inv : 0.f;
             }
-            __builtin_amdgcn_wave_barrier();
-            nrc_backward_tile(w, s, gl, rt, lane);
-            if ((lane >> 4) == rt && valid) nrc_encode_backward(v, p, s.dx + (lane & 15) * (kNrcIn + 1));
-            __builtin_amdgcn_wave_barrier();
         }
+        __builtin_amdgcn_wave_barrier();
+        // output layer: dW4[k][c] = sum_rows h3[row][k] dy[row][c]; G3 = dy W4^T x relu'(h3)
+#pragma unroll 4
+        for (int row = 0; row < 16; ++row) {
+            const float hv = bf2f(s.h[2][row * kHs + lane]);
+            const float y0 = s.y[row * 4], y1 = s.y[row * 4 + 1], y2 = s.y[row * 4 + 2];
+            g4[0] += hv * y0;
+            g4[1] += hv * y1;
+            g4[2] += hv * y2;
+            const float gs = y0 * w4r[0] + y1 * w4r[1] + y2 * w4r[2];
+            s.h[2][row * kHs + lane] = f2bf(hv > 0.f ? gs : 0.f);
+        }
+        __builtin_amdgcn_wave_barrier();
+        nrc_weight_grad<kNrcHidden>(s.h[1], kHs, s.h[2], g3, lane);             // dW3 = H2^T G3
+        __builtin_amdgcn_wave_barrier();
+        nrc_input_grad<kNrcHidden>(s.h[2], wb.w3, s.h[1], nullptr, 0u, lane);   // G2
+        __builtin_amdgcn_wave_barrier();
+        nrc_weight_grad<kNrcHidden>(s.h[0], kHs, s.h[1], g2, lane);             // dW2 = H1^T G2
+        __builtin_amdgcn_wave_barrier();
+        nrc_input_grad<kNrcHidden>(s.h[1], wb.w2, s.h[0], nullptr, 0u, lane);   // G1
+        __builtin_amdgcn_wave_barrier();
+        nrc_weight_grad<kNrcIn>(s.x, kXs, s.h[0], g1, lane);                    // dW1 = X^T G1
+        nrc_input_grad<kNrcIn>(s.h[0], wb.w1, nullptr, dx + size_t(base - first) * kNrcIn, present, lane);// dX
+        __builtin_amdgcn_wave_barrier();
     }
-    // loss: wave sum, one atomic per wave
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off);
-    if (lane == 0 && loss_acc != 0.f) atomicAdd(loss, loss_acc);
     __syncthreads();
-    for (int i = threadIdx.x; i < kNrcIn * kNrcHidden; i += kBlock)
-        if (gl.w1[i] != 0.f) atomicAdd(v.mlp_g + kNrcW1 + i, gl.w1[i]);
-    for (int i = threadIdx.x; i < kNrcHidden * kNrcHidden; i += kBlock) {
-        if (gl.w2[i] != 0.f) atomicAdd(v.mlp_g + kNrcW2 + i, gl.w2[i]);
-        if (gl.w3[i] != 0.f) atomicAdd(v.mlp_g + kNrcW3 + i, gl.w3[i]);
+    NrcGradLds &gl = sh.grad;
+    float *flat = gl.w1;
+    for (int i = threadIdx.x; i < kNrcPartial; i += kBackBlock) flat[i] = 0.f;
+    __syncthreads();
+    if (lane == 0) atomicAdd(&sh.grad.loss, loss_acc);
+    nrc_add_weight_grad<kNrcIn>(g1, gl.w1, lane);
+    nrc_add_weight_grad<kNrcHidden>(g2, gl.w2, lane);
+    nrc_add_weight_grad<kNrcHidden>(g3, gl.w3, lane);
+    for (int c = 0; c < 3; ++c) atomicAdd(gl.w4 + lane * 3 + c, g4[c]);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kNrcPartial; i += kBackBlock) partial[i] = flat[i];
+}
+
+// the blocks' weight gradients and losses added to v.mlp_g and *loss: 32
+// parameters a block, eight lanes' sums each
+__global__ void __launch_bounds__(kBlock) nrc_reduce_kernel(NrcView v, const float *__restrict__ partial,
+                                                            uint32_t blocks, float *__restrict__ loss) {
+    __shared__ float sum[8][32];
+    const uint32_t c = threadIdx.x & 31u, part = threadIdx.x >> 5, i = blockIdx.x * 32u + c;
+    float acc = 0.f;
+    if (i < uint32_t(kNrcPartial)) {
+#pragma unroll 8
+        for (uint32_t b = part; b < blocks; b += 8u) acc += partial[size_t(b) * kNrcPartial + i];
     }
-    for (int i = threadIdx.x; i < kNrcHidden * kNrcOut; i += kBlock)
-        if (gl.w4[i] != 0.f) atomicAdd(v.mlp_g + kNrcW4 + i, gl.w4[i]);
+    sum[part][c] = acc;
+    __syncthreads();
+    if (part == 0 && i < uint32_t(kNrcPartial)) {
+        for (int k = 1; k < 8; ++k) acc += sum[k][c];
+        if (i < uint32_t(kNrcMlpParams)) v.mlp_g[i] += acc;
+        else *loss += acc;
+    }
+}
+
+// The features' gradients dx[row - first][32] into the grid's.  Lane = row 4 x
+// corner 8 x feature 2: a corner's two features, and mostly the corners along
+// x, are neighbours in memory, so the 64 atomics of an instruction touch some
+// 20 lines, and the atomics, which are carried out at the memory side, bound
+// this.  Each wave starts at a level of its own, which spreads the atomics on
+// the few entries of the coarse levels over time.
+__global__ void __launch_bounds__(kBlock) nrc_scatter_kernel(NrcView v, const NrcSample *__restrict__ samples,
+                                                             const uint32_t *__restrict__ count, uint32_t cap,
+                                                             uint32_t offset, uint32_t batch, uint32_t first,
+                                                             uint32_t span, const float *__restrict__ dx) {
+    __shared__ uint32_t res[kNrcLevels];
+    if (threadIdx.x < kNrcLevels) res[threadIdx.x] = v.res[threadIdx.x];
+    __syncthreads();
+    const uint32_t n = nrc_rows(count, cap, offset, batch);
+    const uint32_t end = min(n, first + span);
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = blockIdx.x * (kBlock / 64) + threadIdx.x / 64;
+    const uint32_t row = first + wave * 4u + uint32_t(lane >> 4);
+    if (row >= end) return;
+    const int ft = lane & 1, k = (lane >> 1) & 7;
+    float u[3];
+    nrc_unit(v, samples[offset + row].p, u);
+    const float *d = dx + size_t(row - first) * kNrcIn;
+#pragma unroll 4
+    for (int i = 0; i < kNrcLevels; ++i) {
+        const int l = (i + int(wave)) & (kNrcLevels - 1);
+        const float d0 = d[2 * l], d1 = d[2 * l + 1];
+        if (d0 == 0.f && d1 == 0.f) continue;
+        uint32_t c[3];
+        float f[3];
+        nrc_cell(res[l], u, c, f);
+        float *gg = v.grid_g + size_t(l) * kNrcTable * kNrcFeatures;
+        const uint32_t idx = nrc_index((v.dense_mask >> l) & 1u, res[l], c[0] + (k & 1), c[1] + ((k >> 1) & 1),
+                                       c[2] + ((k >> 2) & 1));
+        atomicAdd(gg + 2 * idx + ft, nrc_corner_weight(k, f) * (ft ? d1 : d0));
+    }
 }
 
 __device__ __forceinline__ float adam_update(float &p, float &m, float &vv, float &g, float lr, float c1, float c2) {
@@ -192,14 +344,24 @@ __device__ __forceinline__ float adam_update(float &p, float &m, float &vv, floa
     return p;
 }
 
+// blockIdx.y: a level of the grid, or the network's weights.  Bound by HBM (34 B
+// a parameter); the tail of a directly indexed level's table, which no position
+// reaches, has no gradient and no moments and is left out (27 % of the table at
+// the default resolutions: 112 -> 80 us a step)
 __global__ void __launch_bounds__(256) nrc_adam_kernel(NrcView v, float lr, float c1, float c2) {
     const size_t stride = size_t(gridDim.x) * blockDim.x;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < kNrcGridParams + kNrcMlpParams; i += stride) {
-        if (i < kNrcGridParams) {
+    const uint32_t l = blockIdx.y;
+    if (l < uint32_t(kNrcLevels)) {
+        const size_t n1 = v.res[l] + 1u;
+        const size_t used = ((v.dense_mask >> l) & 1u ? n1 * n1 * n1 : size_t(kNrcTable)) * kNrcFeatures;
+        const size_t base = size_t(l) * kNrcTable * kNrcFeatures;
+        for (size_t k = size_t(blockIdx.x) * blockDim.x + threadIdx.x; k < used; k += stride) {
+            const size_t i = base + k;
             float p = adam_update(v.grid[i], v.grid_m[i], v.grid_v[i], v.grid_g[i], lr, c1, c2);
             v.grid_f16[i] = f2h(p);
-        } else {
-            size_t j = i - kNrcGridParams;
+        }
+    } else {
+        for (size_t j = size_t(blockIdx.x) * blockDim.x + threadIdx.x; j < kNrcMlpParams; j += stride) {
             float p = adam_update(v.mlp[j], v.mlp_m[j], v.mlp_v[j], v.mlp_g[j], lr, c1, c2);
             v.mlp_bf16[j] = f2bf(p);
         }
@@ -422,34 +584,80 @@ uint32_t grid_blocks() {
 
 }// namespace
 
-hipError_t nrc_forward(const NrcView &v, const float *pos, uint32_t n, float *out, hipStream_t s) {
-    if (!n) return hipSuccess;
-    uint32_t blocks = std::min<uint32_t>((n + kBlock - 1) / kBlock, 8u * grid_blocks());
-    hipLaunchKernelGGL(nrc_forward_kernel<false>, dim3(blocks), dim3(kBlock), 0, s, v, pos, n, nullptr, nullptr, 0u,
-                       out, nullptr);
+namespace {
+
+// features of rows [first, first + span), sixteen rows a lane from half a
+// million on: 1 M rows took 437 us at one row a lane, 381 at four, 344 at eight
+// and 270 at sixteen (a wave a SIMD), 65536 rows 29 us at one
+hipError_t encode(const NrcView &v, const float *pos, uint32_t stride, const uint32_t *count, uint32_t cap,
+                  uint32_t offset, uint32_t batch, uint32_t first, uint32_t span, uint32_t *feat, hipStream_t s) {
+    if (span >= (1u << 19))
+        hipLaunchKernelGGL(nrc_encode_kernel<16>, dim3((span + kBlock * 16 - 1) / (kBlock * 16)), dim3(kBlock), 0, s, v,
+                           pos, stride, count, cap, offset, batch, first, span, feat);
+    else
+        hipLaunchKernelGGL(nrc_encode_kernel<1>, dim3((span + kBlock - 1) / kBlock), dim3(kBlock), 0, s, v, pos,
+                           stride, count, cap, offset, batch, first, span, feat);
     return hipGetLastError();
+}
+
+uint32_t forward_blocks(uint32_t span) { return std::min<uint32_t>((span + kBlock - 1) / kBlock, 8u * grid_blocks()); }
+
+}// namespace
+
+hipError_t nrc_forward(const NrcView &v, const float *pos, uint32_t n, float *out, const NrcScratch &sc,
+                       hipStream_t s) {
+    for (uint32_t first = 0; first < n; first += sc.rows) {
+        const uint32_t span = std::min(sc.rows, n - first);
+        hipError_t e = encode(v, pos, 3, nullptr, n, 0, n, first, span, sc.feat, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(nrc_forward_kernel<false>, dim3(forward_blocks(span)), dim3(kBlock), 0, s, v, sc.feat,
+                           nullptr, nullptr, n, first, span, out, nullptr);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t nrc_infer(const NrcView &v, const NrcQuery *q, const uint32_t *count, uint32_t capacity, float4 *L,
-                     hipStream_t s) {
-    if (!capacity) return hipSuccess;
-    uint32_t blocks = std::min<uint32_t>((capacity + kBlock - 1) / kBlock, 8u * grid_blocks());
-    hipLaunchKernelGGL(nrc_forward_kernel<true>, dim3(blocks), dim3(kBlock), 0, s, v, nullptr, 0u, q, count,
-                       capacity, nullptr, L);
-    return hipGetLastError();
+                     const NrcScratch &sc, hipStream_t s) {
+    static_assert(sizeof(NrcQuery) == 32 && offsetof(NrcQuery, p) == 0, "query layout");
+    for (uint32_t first = 0; first < capacity; first += sc.rows) {
+        const uint32_t span = std::min(sc.rows, capacity - first);
+        hipError_t e = encode(v, q->p, 8, count, capacity, 0, capacity, first, span, sc.feat, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(nrc_forward_kernel<true>, dim3(forward_blocks(span)), dim3(kBlock), 0, s, v, sc.feat, q,
+                           count, capacity, first, span, nullptr, L);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
+uint32_t nrc_backward_blocks() { return grid_blocks(); }
+
 hipError_t nrc_backward(const NrcView &v, const NrcSample *samples, const uint32_t *count, uint32_t capacity,
-                        uint32_t offset, uint32_t batch, float *loss, uint32_t blocks, hipStream_t s) {
-    if (!capacity || !batch) return hipSuccess;
-    if (!blocks) blocks = grid_blocks();
-    hipLaunchKernelGGL(nrc_backward_kernel, dim3(blocks), dim3(kBlock), 0, s, v, samples, count, capacity, offset,
-                       batch, loss);
-    return hipGetLastError();
+                        uint32_t offset, uint32_t batch, float *loss, const NrcScratch &sc, hipStream_t s) {
+    static_assert(sizeof(NrcSample) == 24 && offsetof(NrcSample, p) == 0, "sample layout");
+    const uint32_t rows = std::min(batch, capacity);
+    for (uint32_t first = 0; first < rows; first += sc.rows) {
+        const uint32_t span = std::min(sc.rows, rows - first);
+        hipError_t e = encode(v, samples->p, 6, count, capacity, offset, batch, first, span, sc.feat, s);
+        if (e != hipSuccess) return e;
+        const uint32_t blocks = std::min((span + kBackWaves * 16 - 1) / (kBackWaves * 16), grid_blocks());
+        hipLaunchKernelGGL(nrc_backward_kernel, dim3(blocks), dim3(kBackBlock), 0, s, v, samples, sc.feat, count,
+                           capacity, offset, batch, first, span, sc.dx, sc.partial);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(nrc_reduce_kernel, dim3((kNrcPartial + 31) / 32), dim3(kBlock), 0, s, v, sc.partial, blocks,
+                           loss);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        const uint32_t per = 4u * (kBlock / 64);
+        hipLaunchKernelGGL(nrc_scatter_kernel, dim3((span + per - 1) / per), dim3(kBlock), 0, s, v, samples, count,
+                           capacity, offset, batch, first, span, sc.dx);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t nrc_adam(const NrcView &v, float lr, float c1, float c2, hipStream_t s) {
-    hipLaunchKernelGGL(nrc_adam_kernel, dim3(8u * grid_blocks()), dim3(256), 0, s, v, lr, c1, c2);
+    hipLaunchKernelGGL(nrc_adam_kernel, dim3(grid_blocks(), kNrcLevels + 1), dim3(256), 0, s, v, lr, c1, c2);
     return hipGetLastError();
 }
 
