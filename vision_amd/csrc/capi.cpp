@@ -700,13 +700,18 @@ bool vs_internal::wavefront_reserve(WavefrontBuffers &wb, size_t cap) {
         hip_check(hipHostMalloc(&hp, 64, hipHostMallocDefault), "pinned counts");
         wb.host_counts = static_cast<uint32_t *>(hp);
     }
+    if (!wb.ev_count) hip_check(hipEventCreateWithFlags(&wb.ev_count, hipEventDisableTiming), "event");
     wb.capacity = 0;
     DevBuf *all[] = {&wb.o, &wb.d, &wb.thr, &wb.L, &wb.meta, &wb.lam, &wb.lpdf, &wb.hit, &wb.sh_o, &wb.sh_d, &wb.sh_c,
                      &wb.q0, &wb.q1, &wb.counts};
     for (DevBuf *b : all) b->release();
     try {
-        for (DevBuf *b : all)
-            b->alloc(b == &wb.counts ? 64 : (b == &wb.q0 || b == &wb.q1 ? cap * 4 : cap * 16));
+        const size_t queue = vs::wf_queue_capacity(cap);
+        for (DevBuf *b : all) {
+            if (b == &wb.counts) b->alloc(vs::kWfWords * 4);
+            else if (b == &wb.q0 || b == &wb.q1) b->alloc(queue * 4);
+            else b->alloc((b == &wb.sh_o || b == &wb.sh_d || b == &wb.sh_c ? queue : cap) * 16);
+        }
     } catch (const DeviceError &) {
         for (DevBuf *b : all) b->release();
         return false;
@@ -720,7 +725,7 @@ uint32_t vs_internal::wavefront_render(const vs::SceneView &view, const vs::Came
                                        float4 *out,
                                        uint32_t frame_index, uint32_t spp, uint32_t chunk_frames,
                                        uint32_t trace_block, WavefrontBuffers &wb, hipStream_t st,
-                                       unsigned long long *ctr, vs_render_stats *ts, hipEvent_t *ev) {
+                                       unsigned long long *ctr, vs_render_stats *ts) {
     const uint32_t P = cam.width * cam.height;
     const uint32_t chunk = std::min<uint32_t>(chunk_frames, spp);
     const size_t cap = size_t(P) * chunk;
@@ -743,44 +748,62 @@ uint32_t vs_internal::wavefront_render(const vs::SceneView &view, const vs::Came
     const uint32_t dim = rv0.spectrum_dim;
     uint32_t *q[2] = {wb.q0.as<uint32_t>(), wb.q1.as<uint32_t>()};
     uint32_t *counts = wb.counts.as<uint32_t>();
-    const bool timed = ts && ev;
-    uint32_t launches = 0;
+    size_t stamps = 0;
+    auto stamp = [&] {
+        if (!ts) return;
+        if (stamps == wb.ev.size()) {
+            hipEvent_t e = nullptr;
+            hip_check(hipEventCreate(&e), "event");
+            wb.ev.push_back(e);
+        }
+        hip_check(hipEventRecord(wb.ev[stamps++], st), "event");
+    };
+    uint32_t launches = 1;
+    hip_check(vs::wf_zero(counts, st), "wf zero");
     for (uint32_t f0 = 0; f0 < spp; f0 += chunk) {
         const uint32_t fc = std::min(chunk, spp - f0);
         const uint32_t n = P * fc;
         const uint32_t frame0 = frame_index + f0;
-        hip_check(vs::wf_begin(cam, rv0, w, dim, rgb, frame0, n, q[0], st), "wf begin");
+        hip_check(vs::wf_begin(cam, rv0, w, dim, rgb, frame0, n, st), "wf begin");
         ++launches;
         uint32_t count = rv0.max_depth > 0 ? n : 0u;
+        vs::WavefrontQueue queue{nullptr, counts + vs::kWfLiveFirst, 0u};// the first bounce: every path
         int cur = 0;
         while (count) {
-            hip_check(vs::wf_zero(counts, st), "wf zero");
-            if (timed) hip_check(hipEventRecord(ev[0], st), "event");
-            hip_check(vs::wf_trace(view, w, q[cur], count, ctr, trace_block, st), "wf trace");
-            if (timed) hip_check(hipEventRecord(ev[1], st), "event");
-            hip_check(vs::wf_shade(view, rv0, w, dim, rgb, diffuse_only ? 1 : 0, q[cur], count, q[cur ^ 1], counts, st), "wf shade");
-            if (timed) hip_check(hipEventRecord(ev[2], st), "event");
-            hip_check(vs::wf_shadow(view, w, counts, count, ctr ? ctr + 4 : nullptr, trace_block, st), "wf shadow");
-            if (timed) hip_check(hipEventRecord(ev[3], st), "event");
+            const uint32_t segment = vs::wf_segment(count);
+            stamp();
+            hip_check(vs::wf_trace(view, w, queue, count, ctr, trace_block, st), "wf trace");
+            stamp();
+            hip_check(vs::wf_shade(view, rv0, w, dim, rgb, diffuse_only ? 1 : 0, queue, count, q[cur], counts, st), "wf shade");
+            stamp();
+            hip_check(vs::wf_fold(counts, st), "wf fold");
+            hip_check(hipMemcpyAsync(wb.host_counts, counts + vs::kWfLiveFirst + vs::kWfSegments, 4,
+                                     hipMemcpyDeviceToHost, st),
+                      "wf counts");
+            hip_check(hipEventRecord(wb.ev_count, st), "event");
+            hip_check(vs::wf_shadow(view, w, counts, count, segment, ctr ? ctr + 4 : nullptr, trace_block, st), "wf shadow");
+            stamp();
             launches += 4;
-            hip_check(hipMemcpyAsync(wb.host_counts, counts, 8, hipMemcpyDeviceToHost, st), "wf counts");
-            hip_check(hipStreamSynchronize(st), "wf sync");
-            if (timed) {
-                float t_trace = 0.f, t_shade = 0.f, t_shadow = 0.f;
-                hip_check(hipEventElapsedTime(&t_trace, ev[0], ev[1]), "event time");
-                hip_check(hipEventElapsedTime(&t_shade, ev[1], ev[2]), "event time");
-                hip_check(hipEventElapsedTime(&t_shadow, ev[2], ev[3]), "event time");
-                ts->stage_ms[0] += t_trace;
-                ts->stage_ms[1] += t_shade;
-                ts->stage_ms[2] += t_shadow;
-                for (int k = 0; k < 3; ++k) ts->stage_launches[k] += 1;
-            }
-            count = wb.host_counts[vs::WF_LIVE];
+            // the any-hit rays run while the host takes the count
+            hip_check(hipEventSynchronize(wb.ev_count), "wf sync");
+            queue.items = q[cur];
+            queue.segment = segment;
+            count = *wb.host_counts;
             if (count > n) throw std::logic_error("wavefront queue overflow");
             cur ^= 1;
         }
         hip_check(vs::wf_accumulate(rv0, w, frame0, fc, rt, out, st), "wf accumulate");
         ++launches;
+    }
+    if (ts) {
+        hip_check(hipStreamSynchronize(st), "wf sync");
+        for (size_t b = 0; b + 3 < stamps; b += 4)
+            for (int k = 0; k < 3; ++k) {
+                float ms = 0.f;
+                hip_check(hipEventElapsedTime(&ms, wb.ev[b + k], wb.ev[b + k + 1]), "event time");
+                ts->stage_ms[k] += ms;
+                ts->stage_launches[k] += 1;
+            }
     }
     return launches;
 }
@@ -792,11 +815,10 @@ namespace {
 // Wavefront render of `spp` frames of a scene's film from its frame index
 uint32_t render_wavefront(vs_scene *s, const vs::RenderView &rv0, uint32_t spp, unsigned long long *ctr,
                           vs_render_stats &ts) {
-    hipEvent_t ev[4] = {s->ctx->tr0, s->ctx->tr1, s->ctx->tr2, s->ctx->ev1};
     return wavefront_render(s->view, s->cam, rv0, s->packed.rgb, s->diffuse_only, s->film_rt.as<float4>(),
                             s->film_out.as<float4>(),
                             s->frame_index, spp, s->wf_chunk_frames, s->wf_trace_block, s->wf, s->ctx->stream, ctr,
-                            &ts, ev);
+                            &ts);
 }
 
 // The megakernel form's fused job of several frames, where running a pixel's
@@ -824,7 +846,7 @@ bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, uint32_t &laun
         if (P * chunk > 0xFFFFFFFFull || !wavefront_reserve(s->wf, size_t(P) * chunk)) return false;
         launches += wavefront_render(s->view, s->cam, rv, s->packed.rgb, false, s->film_rt.as<float4>(),
                                      s->film_out.as<float4>(), s->frame_index, spp, chunk, 64, s->wf, s->ctx->stream,
-                                     nullptr, nullptr, nullptr);
+                                     nullptr, nullptr);
         return true;
     }
     if (P > (4u << 20)) return false;

@@ -98,11 +98,15 @@ struct WavefrontBuffers {
     size_t capacity{0};
     DevBuf o, d, thr, L, meta, lam, lpdf, hit, sh_o, sh_d, sh_c, q0, q1, counts;
     uint32_t *host_counts{nullptr};// pinned
+    hipEvent_t ev_count{nullptr};  // the live count is on the host
+    std::vector<hipEvent_t> ev;    // stage times, four a bounce, made as needed
     WavefrontBuffers() = default;
     WavefrontBuffers(const WavefrontBuffers &) = delete;
     WavefrontBuffers &operator=(const WavefrontBuffers &) = delete;
     ~WavefrontBuffers() {
         if (host_counts) (void)hipHostFree(host_counts);
+        if (ev_count) (void)hipEventDestroy(ev_count);
+        for (hipEvent_t e : ev) (void)hipEventDestroy(e);
     }
 };
 
@@ -225,14 +229,14 @@ inline void require_built(vs_scene *s) {
 // The wavefront form over one film: `spp` frames from frame_index in
 // chunks of `chunk` frames, each a loop of trace / shade / shadow over the
 // live-path queue until it empties, then the chunk folds into the film.
-// Synchronises `st` once per bounce (the live count).  Returns launches;
-// adds per-stage times to *ts when it and the three events are given.
+// Waits once per bounce, for the live count.  Returns launches; adds per-stage
+// times to *ts when it is given (then `st` is idle on return).
 // wavefront_reserve: path state for `paths` paths; false (and nothing held)
 // when the device has no room.
 bool wavefront_reserve(WavefrontBuffers &wb, size_t paths);
 uint32_t wavefront_render(const vs::SceneView &view, const vs::CameraView &cam, const vs::RenderView &rv0,
                           bool rgb, bool diffuse_only, float4 *rt, float4 *out, uint32_t frame_index, uint32_t spp, uint32_t chunk,
                           uint32_t trace_block, WavefrontBuffers &wb, hipStream_t st, unsigned long long *ctr,
-                          vs_render_stats *ts, hipEvent_t *ev4);
+                          vs_render_stats *ts);
 
 }// namespace vs_internal

@@ -167,7 +167,6 @@ struct vs_server {
     std::thread lane[kLanes];
     hipStream_t st_lane[kLanes]{};
     WavefrontBuffers lane_wb[kLanes];
-    hipEvent_t lane_ev[kLanes][4]{};// stage timing of each lane's bounces
     DevBuf lane_ctr[kLanes];         // counting runs: 8 counters per lane
     // lane totals (under mu)
     uint64_t lane_samples{0}, lane_stage_launches[3]{}, lane_counts[6]{};
@@ -610,7 +609,7 @@ void lane_main(vs_server *S, int lane) {
             }
             vs_render_stats ts{};
             wavefront_render(view, cam, j->rv, !j->d.spectral, diffuse_only, rt, out, 0, j->d.spp, chunk,
-                             64, S->lane_wb[lane], ls, ctr, &ts, S->lane_ev[lane]);
+                             64, S->lane_wb[lane], ls, ctr, &ts);
             unsigned long long c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             if (ctr) hip_check(hipMemcpyAsync(c, ctr, sizeof(c), hipMemcpyDeviceToHost, ls), "lane counters D2H");
             hip_check(vs::serve_output(j->rv, rt, out, px, ls), "output pass");
@@ -757,10 +756,7 @@ vs_status vs_server_create(vs_context *ctx, const vs_server_config *cfg, vs_serv
         hip_check(hipMemset(S->d_counters.ptr, 0, 8 * sizeof(unsigned long long)), "counter clear");
         S->slot_job.assign(S->cfg.max_jobs, nullptr);
         for (auto &ls : S->st_lane) hip_check(hipStreamCreateWithFlags(&ls, hipStreamNonBlocking), "stream");
-        for (int l = 0; l < vs_server::kLanes; ++l) {
-            for (auto &e : S->lane_ev[l]) hip_check(hipEventCreate(&e), "lane event");
-            S->lane_ctr[l].alloc(8 * sizeof(unsigned long long));
-        }
+        for (DevBuf &c : S->lane_ctr) c.alloc(8 * sizeof(unsigned long long));
         S->worker = std::thread(worker_main, S.get());
         for (int l = 0; l < vs_server::kLanes; ++l) S->lane[l] = std::thread(lane_main, S.get(), l);
     });
@@ -1208,9 +1204,6 @@ void vs_server_destroy(vs_server *S) {
             (void)hipStreamSynchronize(ls);
             (void)hipStreamDestroy(ls);
         }
-        for (auto &evs : S->lane_ev)
-            for (auto &e : evs)
-                if (e) (void)hipEventDestroy(e);
     }
     delete S;
 }
