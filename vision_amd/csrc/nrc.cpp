@@ -72,22 +72,39 @@ void adam_step(vs_nrc *n, hipStream_t st) {
     hip_check(vs::nrc_adam(n->view, n->cfg.learning_rate, c1, c2, st), "adam");
 }
 
-// the kernels' workspace for up to `rows` rows, at most 4 M queries (268 MB of
-// features) or 1 M training samples (200 MB with their gradients) at a time
-vs::NrcScratch scratch(vs_nrc *n, size_t rows, bool backward) {
-    vs::NrcScratch sc{};
-    sc.rows = uint32_t(std::min<size_t>(rows, backward ? 1u << 20 : 4u << 20));
-    const size_t f = size_t(sc.rows) * vs::kNrcLevels * 4, d = size_t(sc.rows) * vs::kNrcIn * sizeof(float);
-    if (n->feat.bytes < f) n->feat.alloc(f);
-    if (backward && n->dx.bytes < d) n->dx.alloc(d);
-    sc.feat = n->feat.as<uint32_t>();
-    sc.dx = n->dx.as<float>();
-    if (backward) {
-        const size_t p = size_t(vs::nrc_backward_blocks()) * vs::kNrcPartial * sizeof(float);
-        if (n->partial.bytes < p) n->partial.alloc(p);
-        sc.partial = n->partial.as<float>();
+// the kernels' workspace, one for both uses: up to 1 M queries (67 MB of
+// features) or training samples (200 MB with their gradients) at a time, and
+// fewer where the device has no room for that.  1 M queries' features stay in
+// the last-level cache between the encoding and the network: 4 frames of 8.3 M
+// query slots take 4.62 ms, with 4 M at a time 5.65, with 256 K (more launches)
+// 7.22.
+struct Workspace {
+    vs::NrcScratch infer{}, train{};
+};
+
+Workspace scratch(vs_nrc *n, size_t queries, size_t samples) {
+    Workspace w;
+    w.infer.rows = uint32_t(std::min<size_t>(queries, 1u << 20));
+    w.train.rows = uint32_t(std::min<size_t>(samples, 1u << 20));
+    for (;;) {
+        const size_t f = size_t(std::max(w.infer.rows, w.train.rows)) * vs::kNrcLevels * 4;
+        const size_t d = size_t(w.train.rows) * vs::kNrcIn * sizeof(float);
+        try {
+            if (n->feat.bytes < f) n->feat.alloc(f);
+            if (n->dx.bytes < d) n->dx.alloc(d);
+            break;
+        } catch (const DeviceError &) {
+            if (std::max(w.infer.rows, w.train.rows) <= 65536u) throw;
+            w.infer.rows = std::min(w.infer.rows, std::max(w.infer.rows / 2u, 65536u));
+            w.train.rows = std::min(w.train.rows, std::max(w.train.rows / 2u, 65536u));
+        }
     }
-    return sc;
+    const size_t p = size_t(vs::nrc_backward_blocks()) * vs::kNrcPartial * sizeof(float);
+    if (w.train.rows && n->partial.bytes < p) n->partial.alloc(p);
+    w.infer.feat = w.train.feat = n->feat.as<uint32_t>();
+    w.train.dx = n->dx.as<float>();
+    w.train.partial = n->partial.as<float>();
+    return w;
 }
 
 uint32_t train_stride(const vs_nrc *n, uint32_t pixels) {
@@ -240,7 +257,7 @@ vs_status vs_nrc_forward(vs_nrc *n, const float *pos, uint32_t count, float *out
         if (n->io_a.bytes < size_t(count) * 12) n->io_a.alloc(size_t(count) * 12);
         if (n->io_b.bytes < size_t(count) * 12) n->io_b.alloc(size_t(count) * 12);
         hip_check(hipMemcpyAsync(n->io_a.ptr, pos, size_t(count) * 12, hipMemcpyHostToDevice, st), "pos H2D");
-        hip_check(vs::nrc_forward(n->view, n->io_a.as<float>(), count, n->io_b.as<float>(), scratch(n, count, false), st), "forward");
+        hip_check(vs::nrc_forward(n->view, n->io_a.as<float>(), count, n->io_b.as<float>(), scratch(n, count, 0).infer, st), "forward");
         hip_check(hipMemcpyAsync(out, n->io_b.ptr, size_t(count) * 12, hipMemcpyDeviceToHost, st), "out D2H");
         hip_check(hipStreamSynchronize(st), "sync");
     });
@@ -259,7 +276,7 @@ vs_status vs_nrc_gradients(vs_nrc *n, const float *samples, uint32_t count, floa
         hip_check(hipMemsetAsync(n->mlp_g.ptr, 0, sizeof(float) * vs::kNrcMlpParams, st), "clear");
         hip_check(hipMemsetAsync(n->grid_g.ptr, 0, sizeof(float) * vs::kNrcGridParams, st), "clear");
         hip_check(vs::nrc_backward(n->view, n->io_a.as<vs::NrcSample>(), n->counts.as<uint32_t>(), count, 0, count,
-                                   n->loss.as<float>(), scratch(n, count, true), st),
+                                   n->loss.as<float>(), scratch(n, 0, count).train, st),
                   "backward");
         hip_check(hipMemcpyAsync(loss, n->loss.ptr, 4, hipMemcpyDeviceToHost, st), "loss D2H");
         hip_check(hipMemcpyAsync(mlp_grad, n->mlp_g.ptr, sizeof(float) * vs::kNrcMlpParams, hipMemcpyDeviceToHost, st),
@@ -282,7 +299,7 @@ vs_status vs_nrc_train(vs_nrc *n, const float *samples, uint32_t count, uint32_t
         if (n->io_a.bytes < size_t(count) * 24) n->io_a.alloc(size_t(count) * 24);
         hip_check(hipMemcpyAsync(n->io_a.ptr, samples, size_t(count) * 24, hipMemcpyHostToDevice, st), "H2D");
         hip_check(hipMemcpyAsync(n->counts.ptr, &count, 4, hipMemcpyHostToDevice, st), "count");
-        const vs::NrcScratch sc = scratch(n, count, true);
+        const vs::NrcScratch sc = scratch(n, 0, count).train;
         for (uint32_t i = 0; i < steps; ++i) {
             hip_check(hipMemsetAsync(n->loss.ptr, 0, 4, st), "loss clear");
             hip_check(vs::nrc_backward(n->view, n->io_a.as<vs::NrcSample>(), n->counts.as<uint32_t>(), count, 0,
@@ -327,13 +344,8 @@ vs_status vs_nrc_render(vs_nrc *n, uint32_t frames, uint32_t spp, uint32_t flags
             n->staging_paths = paths;
             n->sample_cap = paths * maxv;
         }
-        // one workspace for both: the larger of the two is allocated first
         const uint32_t train_rows = n->cfg.train_batch ? std::min(n->cfg.train_batch, n->sample_cap) : n->sample_cap;
-        vs::NrcScratch infer_sc{}, train_sc{};
-        for (int pass = 0; pass < 2; ++pass) {
-            if (terminate) infer_sc = scratch(n, slots, false);
-            if (train) train_sc = scratch(n, std::max(train_rows, 1u), true);
-        }
+        const Workspace work = scratch(n, terminate ? slots : 0, train ? std::max(train_rows, 1u) : 0);
         uint32_t *qcount = n->counts.as<uint32_t>(), *tcount = qcount + 1;
         float ms[6] = {0, 0, 0, 0, 0, 0};
         while (n->fev.size() < size_t(frames) * 6) {
@@ -359,7 +371,7 @@ vs_status vs_nrc_render(vs_nrc *n, uint32_t frames, uint32_t spp, uint32_t flags
             hip_check(hipEventRecord(ev[2], st), "event");
             if (terminate)
                 hip_check(vs::nrc_infer(n->view, n->queries.as<vs::NrcQuery>(), qcount, uint32_t(slots),
-                                        n->L.as<float4>(), infer_sc, st),
+                                        n->L.as<float4>(), work.infer, st),
                           "infer");
             hip_check(hipEventRecord(ev[3], st), "event");
             if (train) {
@@ -370,7 +382,7 @@ vs_status vs_nrc_render(vs_nrc *n, uint32_t frames, uint32_t spp, uint32_t flags
                     const uint32_t off = n->cfg.train_batch ? k * batch : 0u;// wrapped by the kernel
                     hip_check(hipMemsetAsync(n->loss.ptr, 0, 4, st), "loss clear");
                     hip_check(vs::nrc_backward(n->view, n->samples.as<vs::NrcSample>(), tcount, n->sample_cap, off,
-                                               batch, n->loss.as<float>(), train_sc, st),
+                                               batch, n->loss.as<float>(), work.train, st),
                               "backward");
                     adam_step(n, st);
                 }

@@ -606,8 +606,8 @@ uint32_t forward_blocks(uint32_t span) { return std::min<uint32_t>((span + kBloc
 
 hipError_t nrc_forward(const NrcView &v, const float *pos, uint32_t n, float *out, const NrcScratch &sc,
                        hipStream_t s) {
-    for (uint32_t first = 0; first < n; first += sc.rows) {
-        const uint32_t span = std::min(sc.rows, n - first);
+    for (uint32_t first = 0, span; first < n; first += span) {
+        span = std::min(sc.rows, n - first);
         hipError_t e = encode(v, pos, 3, nullptr, n, 0, n, first, span, sc.feat, s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(nrc_forward_kernel<false>, dim3(forward_blocks(span)), dim3(kBlock), 0, s, v, sc.feat,
@@ -620,8 +620,8 @@ hipError_t nrc_forward(const NrcView &v, const float *pos, uint32_t n, float *ou
 hipError_t nrc_infer(const NrcView &v, const NrcQuery *q, const uint32_t *count, uint32_t capacity, float4 *L,
                      const NrcScratch &sc, hipStream_t s) {
     static_assert(sizeof(NrcQuery) == 32 && offsetof(NrcQuery, p) == 0, "query layout");
-    for (uint32_t first = 0; first < capacity; first += sc.rows) {
-        const uint32_t span = std::min(sc.rows, capacity - first);
+    for (uint32_t first = 0, span; first < capacity; first += span) {
+        span = std::min(sc.rows, capacity - first);
         hipError_t e = encode(v, q->p, 8, count, capacity, 0, capacity, first, span, sc.feat, s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(nrc_forward_kernel<true>, dim3(forward_blocks(span)), dim3(kBlock), 0, s, v, sc.feat, q,
@@ -637,8 +637,8 @@ hipError_t nrc_backward(const NrcView &v, const NrcSample *samples, const uint32
                         uint32_t offset, uint32_t batch, float *loss, const NrcScratch &sc, hipStream_t s) {
     static_assert(sizeof(NrcSample) == 24 && offsetof(NrcSample, p) == 0, "sample layout");
     const uint32_t rows = std::min(batch, capacity);
-    for (uint32_t first = 0; first < rows; first += sc.rows) {
-        const uint32_t span = std::min(sc.rows, rows - first);
+    for (uint32_t first = 0, span; first < rows; first += span) {
+        span = std::min(sc.rows, rows - first);
         hipError_t e = encode(v, samples->p, 6, count, capacity, offset, batch, first, span, sc.feat, s);
         if (e != hipSuccess) return e;
         const uint32_t blocks = std::min((span + kBackWaves * 16 - 1) / (kBackWaves * 16), grid_blocks());
