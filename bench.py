@@ -34,8 +34,8 @@ writes, cache hits included):
       kernel is the one of the persistent kernel and the three lane stages
       with the most event time);
   wavefront closest-hit: traversal;
-  wavefront shading: SHADE_BYTES per shaded path (path state in / out,
-      hit, queues, triangle, vertices, instance, material, light sample)
+  wavefront shading: SHADE_BYTES per shaded path (path state 96 in,
+      64 + 32 out, hit, queues, triangle, vertices, instance, material, light)
       + 48 B per shadow ray written;
   wavefront any-hit: traversal + 32 B per shadow ray (contribution, radiance);
   ReSTIR shader0: traversal + 4 x 48 B records (surface and reservoir
@@ -67,7 +67,7 @@ RECORD_BYTES = 48      # ReSTIR surface / reservoir record
 SURFACE_GATHER = 124   # triangle indices 12 + positions 36 + normals 36 + uvs 24 + instance 16
 MATERIAL_BYTES = 128
 CANDIDATE_BYTES = 184  # light selection alias 8 + func 4, light record 112, triangle alias 12, triangle 48
-SHADE_BYTES = 240 + 16 + 8 + SURFACE_GATHER + MATERIAL_BYTES + CANDIDATE_BYTES
+SHADE_BYTES = 192 + 16 + 8 + SURFACE_GATHER + MATERIAL_BYTES + CANDIDATE_BYTES
 
 
 SCENE_CACHE = ROOT / "vision_amd" / "_scenes"

@@ -76,8 +76,8 @@ void adam_step(vs_nrc *n, hipStream_t st) {
 // features) or training samples (200 MB with their gradients) at a time, and
 // fewer where the device has no room for that.  1 M queries' features stay in
 // the last-level cache between the encoding and the network: 4 frames of 8.3 M
-// query slots take 4.62 ms, with 4 M at a time 5.65, with 256 K (more launches)
-// 7.22.
+// query slots take 4.6 ms, with 2 M at a time 5.0, with 4 M 5.65; launches of
+// 512 K and 256 K fill less of the device, 7.1 and 7.2.
 struct Workspace {
     vs::NrcScratch infer{}, train{};
 };
