@@ -832,10 +832,10 @@ uint32_t render_wavefront(vs_scene *s, const vs::RenderView &rv0, uint32_t spp, 
 // kWaveSpp samples a pixel on (up to 32 M paths at a time).  Its bounces are
 // launches with a host wait each, so one or two samples are done sooner by the
 // megakernel.  Measured (megakernel / wavefront ms, procedural scene of 80k
-// triangles, depth 16, sRGB) at 1, 2, 3, 4 and 8 samples: 96 x 54 1.3 / 1.9,
-// 2.4 / 2.2, 3.5 / 2.4, 4.7 / 2.6, 9.4 / 2.8; 639 x 361 1.6 / 3.2, 3.2 / 3.4,
-// 4.7 / 3.5, 6.1 / 3.6, 12.1 / 4.1; 1920 x 1080 2.6 / 4.1, 4.9 / 5.1, 7.3 /
-// 6.0, 9.8 / 7.1, 18.7 / 11.0; at depth 3 and with hero wavelengths alike.
+// triangles, depth 16, sRGB) at 1, 2, 3, 4 and 8 samples: 96 x 54 1.3 / 2.1,
+// 2.5 / 2.4, 3.5 / 2.6, 4.7 / 2.7, 9.4 / 3.0; 639 x 361 1.7 / 3.4, 3.2 / 3.6,
+// 4.7 / 3.7, 6.1 / 3.8, 12.1 / 4.2; 1920 x 1080 2.7 / 4.3, 5.1 / 5.2, 7.3 /
+// 6.0, 9.8 / 6.9, 18.7 / 10.5; at depth 3 and with hero wavelengths alike.
 constexpr uint32_t kWaveSpp = 3;
 
 bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, uint32_t &launches) {

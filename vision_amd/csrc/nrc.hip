@@ -57,7 +57,7 @@ __device__ __forceinline__ void fwd_tile(const NrcWeightsLds &w, NrcFwdLds &s, i
 // time: it stays in every XCD's L2, and the coarse ones in L1.  With a row's
 // levels one after the other the gathers missed L2 half the time and ran at
 // the Infinity Cache's bandwidth (7.5 TB/s): a full-HD frame's queries took
-// 1.92 ms, now 1.43 ms (1.08 of them here).
+// 1.92 ms, now 1.15 ms with the network.
 template <int Q>
 __global__ void __launch_bounds__(kBlock) nrc_encode_kernel(NrcView v, const float *__restrict__ pos, uint32_t stride,
                                                             const uint32_t *__restrict__ count, uint32_t cap,

@@ -129,9 +129,7 @@ trace_queue_kernel(SceneView sc, WavefrontView w, WavefrontQueue queue, uint32_t
 }
 
 // Three resident waves per SIMD (168 VGPRs, 250-420 B of scratch per lane):
-// left free the compiler takes 256 VGPRs and one wave.  Measured on the
-// procedural 1080p 64-spp hero-4 job: 2.64 ms per launch free, 2.06 ms at
-// three waves, 2.21 ms at four, 2.61 ms at five.
+// left free the compiler takes 256 VGPRs and one wave (figures at shade_waves).
 // Before shading, a block sorts its paths by what they hit (the miss branch,
 // a material-less surface, or the material's kind) in LDS, so that a wave
 // mostly runs one branch of path_shade; the block's paths stay the same 256
