@@ -19,6 +19,7 @@
 namespace vs {
 namespace dev {
 
+typedef short bf16x2 __attribute__((ext_vector_type(2)));
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 

@@ -27,6 +27,16 @@ __device__ __forceinline__ uint32_t nrc_rows(const uint32_t *count, uint32_t cap
     return min(total - (total ? offset : 0u), batch);
 }
 
+// Between a wave's stores to LDS and its other lanes' loads of them, and back.
+// The hardware carries out a wave's LDS accesses in order; the fences (no
+// instruction at this scope) keep the compiler to it, for which the barrier
+// alone is no memory access.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // per-wave LDS of the forward-only kernels: one 16-row tile at a time
 // (features, two hidden buffers used in turn, outputs), so that twelve
 // waves per CU fit beside the block's weights
@@ -40,13 +50,13 @@ struct NrcFwdLds {
 // layer 2 has read it
 __device__ __forceinline__ void fwd_tile(const NrcWeightsLds &w, NrcFwdLds &s, int lane) {
     nrc_fwd_tile<kNrcIn, kNrcHidden>(s.x, kXs, w.w1t, kXs, s.h[0], lane);
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[0], kHs, w.w2t, kHs, s.h[1], lane);
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[1], kHs, w.w3t, kHs, s.h[0], lane);
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     nrc_out_tile(s.h[0], w.w4, s.y, lane);
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
 }
 
 // Features of the rows [first, first + span) of a list of positions, `stride`
@@ -125,7 +135,7 @@ __global__ void __launch_bounds__(kBlock) nrc_forward_kernel(NrcView v, const ui
                 for (int l = 0; l < kNrcLevels; l += 2)
                     *reinterpret_cast<uint2 *>(s.x + (lane & 15) * kXs + 2 * l) = make_uint2(x[l], x[l + 1]);
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             fwd_tile(w, s, lane);
             if ((lane >> 4) == rt && valid) {
                 const int i = lane & 15;
@@ -143,7 +153,7 @@ __global__ void __launch_bounds__(kBlock) nrc_forward_kernel(NrcView v, const ui
                     out[3 * size_t(row) + 2] = y2;
                 }
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
         }
     }
 }
@@ -214,17 +224,18 @@ __global__ void __launch_bounds__(kBackBlock) nrc_backward_kernel(NrcView v, con
         for (int k = 0; k < kNrcLevels / 4; ++k) {
             const int l = (lane >> 4) * (kNrcLevels / 4) + k;
             const uint32_t f = valid ? feat[size_t(l) * span + (base + i - first)] : 0u;
-            *reinterpret_cast<uint32_t *>(s.x + i * kXs + 2 * l) = f;
+            // a vector type, which may alias: nrc_weight_grad reads the tile as uint16_t
+            *reinterpret_cast<bf16x2 *>(s.x + i * kXs + 2 * l) = __builtin_bit_cast(bf16x2, f);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_fwd_tile<kNrcIn, kNrcHidden>(s.x, kXs, w.w1t, kXs, s.h[0], lane);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[0], kHs, w.w2t, kHs, s.h[1], lane);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_fwd_tile<kNrcHidden, kNrcHidden>(s.h[1], kHs, w.w3t, kHs, s.h[2], lane);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_out_tile(s.h[2], w.w4, s.y, lane);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         if (lane < 16) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -236,7 +247,7 @@ __global__ void __launch_bounds__(kBackBlock) nrc_backward_kernel(NrcView v, con
                 s.y[i * 4 + c] = valid ? 2.f * d / den * inv : 0.f;
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         // output layer: dW4[k][c] = sum_rows h3[row][k] dy[row][c]; G3 = dy W4^T x relu'(h3)
 #pragma unroll 4
         for (int row = 0; row < 16; ++row) {
@@ -248,18 +259,18 @@ __global__ void __launch_bounds__(kBackBlock) nrc_backward_kernel(NrcView v, con
             const float gs = y0 * w4r[0] + y1 * w4r[1] + y2 * w4r[2];
             s.h[2][row * kHs + lane] = f2bf(hv > 0.f ? gs : 0.f);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_weight_grad<kNrcHidden>(s.h[1], kHs, s.h[2], g3, lane);             // dW3 = H2^T G3
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_input_grad<kNrcHidden>(s.h[2], wb.w3, s.h[1], nullptr, 0u, lane);   // G2
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_weight_grad<kNrcHidden>(s.h[0], kHs, s.h[1], g2, lane);             // dW2 = H1^T G2
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_input_grad<kNrcHidden>(s.h[1], wb.w2, s.h[0], nullptr, 0u, lane);   // G1
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nrc_weight_grad<kNrcIn>(s.x, kXs, s.h[0], g1, lane);                    // dW1 = X^T G1
         nrc_input_grad<kNrcIn>(s.h[0], wb.w1, nullptr, dx + size_t(base - first) * kNrcIn, present, lane);// dX
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
     }
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off);
     __syncthreads();
