@@ -116,6 +116,33 @@ extern "C" void *dc_load(const char *text, const char *base) {
     return s;
 }
 
+// rays [n][8] (origin, t_min, direction, t_max) over a triangle soup through
+// build_bvh8 and traverse: triangle (0xFFFFFFFF: none), t, barycentrics
+extern "C" void dc_trace(const float *P, uint32_t np, const uint32_t *T, uint32_t nt, const float *rays, uint32_t n,
+                         int any, uint32_t *tri, float *t, float *bary) {
+    std::vector<f3> p(np);
+    std::vector<u3> tr(nt);
+    std::memcpy(p.data(), P, sizeof(f3) * np);
+    std::memcpy(tr.data(), T, sizeof(u3) * nt);
+    const Bvh8 bvh = build_bvh8(p, tr);
+    SceneView v{};
+    v.nodes = reinterpret_cast<const uint32_t *>(bvh.nodes.data());
+    v.leaf_tris = reinterpret_cast<const float *>(bvh.tris.data());
+    v.stack_size = bvh.max_depth;
+    std::vector<uint2> stack(bvh.max_depth);
+    uint32_t nodes = 0, tris = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const float *r = rays + 8 * size_t(i);
+        const f3 o = mk3(r[0], r[1], r[2]), d = mk3(r[4], r[5], r[6]);
+        const TraceHit h = any ? traverse<true>(v, o, d, r[3], r[7], stack.data(), 1u, nodes, tris)
+                               : traverse<false>(v, o, d, r[3], r[7], stack.data(), 1u, nodes, tris);
+        tri[i] = h.tri;
+        t[i] = h.t;
+        bary[2 * i] = h.b1;
+        bary[2 * i + 1] = h.b2;
+    }
+}
+
 extern "C" void dc_set_camera(void *p, const float *c) {
     auto *s = static_cast<DcScene *>(p);
     CameraView &v = s->cam;

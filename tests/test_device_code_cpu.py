@@ -57,6 +57,7 @@ def _harness():
     h.dc_load.restype = C.c_void_p
     h.dc_load.argtypes = [C.c_char_p, C.c_char_p]
     h.dc_set_camera.argtypes = [C.c_void_p, _f32]
+    h.dc_trace.argtypes = [_f32, C.c_uint32, _u32, C.c_uint32, _f32, C.c_uint32, C.c_int, _u32, _f32, _f32]
     h.dc_render.argtypes = [C.c_void_p, _f32, C.c_uint32, _f32]
     return h
 
@@ -315,3 +316,26 @@ def test_device_restir_gi_source_equals_oracle_moving_camera_near_specular(dc):
     _restir_equal(dev, orc)
     # temporal reuse kept history somewhere
     assert orc.gi_rsv[2, 0, :, 1].max() > 1
+
+
+def _dev_trace(h, P, T, rays, any_hit=False):
+    n = len(rays)
+    tri, t, bary = np.zeros(n, np.uint32), np.zeros(n, np.float32), np.zeros((n, 2), np.float32)
+    h.dc_trace(np.ascontiguousarray(P, np.float32), len(P), np.ascontiguousarray(T, np.uint32), len(T),
+               np.ascontiguousarray(rays, np.float32), n, int(any_hit), tri, t, bary)
+    return tri, t, bary
+
+
+@pytest.mark.parametrize("extent,size", [(1.0, 0.05), (1e18, 1e5), (4e21, 1e4), (2e22, 1e4), (1e25, 1e3),
+                                         (3e33, 1.0), (1e37, 1e-2)])
+def test_traversal_hits_over_the_builder_extents(dc, wide_soup, extent, size):
+    """Triangles spread over an extent, up to the largest that the builder
+    takes: every hit of the brute force is found, also where a step times 2^24
+    times the largest reciprocal direction (1e12) leaves the floats (from about
+    5e21 on)."""
+    P, T, rays = wide_soup(extent, size)
+    got, ref = _dev_trace(dc, P, T, rays), oracle.trace(P, T, rays, bvh=False)
+    assert (ref[0] != 0xFFFFFFFF).mean() > 0.1
+    assert np.array_equal(got[0], ref[0])
+    assert _bits_equal(got[1][ref[0] != 0xFFFFFFFF], ref[1][ref[0] != 0xFFFFFFFF])
+    assert np.array_equal(_dev_trace(dc, P, T, rays, True)[0] != 0xFFFFFFFF, ref[0] != 0xFFFFFFFF)

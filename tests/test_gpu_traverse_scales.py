@@ -80,3 +80,24 @@ def test_hits_equal_brute_force(gpu_ctx, scale, offset, flat):
     any_id, _, _ = oracle.trace(P, T, flat_rays, any_hit=True, bvh=False)
     assert np.array_equal(occ.astype(bool), any_id != MISS)
     sc.close()
+
+
+@pytest.mark.parametrize("extent,size", [(4e21, 1e4), (1e25, 1e3), (3e33, 1.0)])
+def test_hits_over_the_builder_extents(gpu_ctx, wide_soup, extent, size):
+    """Extents at which a node's step is held as a NaN (from 2^65 on)."""
+    P, _, flat_rays = wide_soup(extent, size)
+    with tempfile.TemporaryDirectory() as d:
+        sc = gpu_ctx.load_text(_scene(P, d), base_dir=d)
+        sc.build_accel()
+    ex = sc.export()
+    rays = np.zeros(len(flat_rays), va.RAY_DTYPE)
+    rays["org"], rays["t_min"], rays["dir"], rays["t_max"] = (flat_rays[:, 0:3], flat_rays[:, 3], flat_rays[:, 4:7],
+                                                              flat_rays[:, 7])
+    tri_id, t, _ = oracle.trace(ex["positions"], ex["triangles"], flat_rays, bvh=False)
+    hit = tri_id != MISS
+    assert hit.mean() > 0.1
+    hits = sc.trace_closest(rays)
+    assert np.array_equal(hits["tri"], tri_id)
+    assert np.array_equal(hits["t"][hit], t[hit])
+    assert np.array_equal(sc.trace_any(rays).astype(bool), hit)
+    sc.close()

@@ -152,13 +152,22 @@ void set_byte(uint32_t *w, int word0, int slot, uint32_t v) {
     word = (word & ~(0xFFu << sh)) | ((v & 0xFFu) << sh);
 }
 
+// The upper half of the float 2^24 * step of a biased exponent, for the
+// traversal.  Its slab tests multiply that by a reciprocal direction, which is
+// at most 1e12 (dev_traverse.h, safe_rcp): from a step of 2^65 on the product
+// may leave the floats, and the half is a NaN instead.  The axis' planes are
+// then NaN, which the tests' minima and maxima drop: it culls nothing.
+uint32_t step_half(uint32_t biased) {
+    return biased <= 127u + 64u ? (biased + 24u) << 7 : 0x7FC0u;
+}
+
 // the traversal's node (bvh.h): the same frame and planes, steps and the
 // leaves' triangles in the form it takes them
 Bvh8Node traversal_node(const Bvh8ExportNode &n, uint32_t leaf_mask) {
     Bvh8Node r{};
     std::copy(n.w, n.w + 20, r.w);
     uint32_t step[3];
-    for (int a = 0; a < 3; ++a) step[a] = std::min(((n.w[3] >> (8 * a)) & 0xFFu) + 24u, 254u) << 7;
+    for (int a = 0; a < 3; ++a) step[a] = step_half((n.w[3] >> (8 * a)) & 0xFFu);
     r.w[3] = step[0] | step[1] << 16;
     r.w[6] = leaf_mask | (n.w[3] & 0xFF000000u);
     r.w[7] = step[2] << 16;

@@ -15,7 +15,8 @@ namespace vs {
 // The node the traversal reads (5 x 16 B):
 //  w[0..2]  origin p (float bits)
 //  w[3]     steps of x (low half) and y (high half), w[7] high half: z; a half
-//           is the upper 16 bits of the float 2^24 * step, step = 2^e
+//           is the upper 16 bits of the float 2^24 * step, step = 2^e up to
+//           e = 64; of a NaN above, with which the axis culls nothing
 //  w[4]     child_base: index of the first internal child node
 //  w[5]     tri_base:   index of the first leaf triangle of this node
 //  w[6]     leaf mask: bit 3 s + k set when slot s is a leaf with more than k
