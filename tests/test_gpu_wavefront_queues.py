@@ -31,3 +31,28 @@ def test_queues_hold_every_path(gpu_ctx, tmp_path, kind, size, chunk):
     assert np.array_equal(got[0][0], got[1][0])
     assert got[0][1:] == got[1][1:]
     sc.close()
+
+
+def _resident():
+    with open("/proc/self/statm") as f:
+        return int(f.read().split()[1]) * 4096
+
+
+def test_stage_times_hold_no_more_events_for_longer_jobs(gpu_ctx):
+    """Stage times of a job of thousands of bounces add up within its time, one
+    launch of each stage a bounce, and host memory does not grow with them (an
+    event of its own for each stamp would be some 60 000 here)."""
+    sc = gpu_ctx.load_text(scenegen.cornell_box(64, 64, max_depth=8, min_depth=8))
+    sc.build_accel()
+    sc.set_resolution(3, 3)
+    sc.set_kernel("wavefront", chunk_frames=1)
+    sc.render(16)
+    before = _resident()
+    sc.render(2000)
+    grown = _resident() - before
+    st = sc.stats()
+    bounces = st["stage_launches"][0]
+    assert 2000 < bounces <= 2000 * 8 and st["stage_launches"] == [bounces] * 3
+    assert all(ms > 0 for ms in st["stage_ms"]) and sum(st["stage_ms"]) < st["kernel_ms"]
+    assert grown < 4 << 20
+    sc.close()

@@ -748,15 +748,24 @@ uint32_t vs_internal::wavefront_render(const vs::SceneView &view, const vs::Came
     const uint32_t dim = rv0.spectrum_dim;
     uint32_t *q[2] = {wb.q0.as<uint32_t>(), wb.q1.as<uint32_t>()};
     uint32_t *counts = wb.counts.as<uint32_t>();
-    size_t stamps = 0;
+    // a bounce's four stamps are read once the next one's count is on the host
+    // (its stages are through by then), and their events used again
+    uint32_t stamps = 0, read = 0;
     auto stamp = [&] {
         if (!ts) return;
-        if (stamps == wb.ev.size()) {
-            hipEvent_t e = nullptr;
-            hip_check(hipEventCreate(&e), "event");
-            wb.ev.push_back(e);
+        hipEvent_t &e = wb.ev[stamps % 8u];
+        if (!e) hip_check(hipEventCreate(&e), "event");
+        hip_check(hipEventRecord(e, st), "event");
+        ++stamps;
+    };
+    auto read_stamps = [&] {
+        for (int k = 0; k < 3; ++k) {
+            float ms = 0.f;
+            hip_check(hipEventElapsedTime(&ms, wb.ev[(read + k) % 8u], wb.ev[(read + k + 1) % 8u]), "event time");
+            ts->stage_ms[k] += ms;
+            ts->stage_launches[k] += 1;
         }
-        hip_check(hipEventRecord(wb.ev[stamps++], st), "event");
+        read += 4;
     };
     uint32_t launches = 1;
     hip_check(vs::wf_zero(counts, st), "wf zero");
@@ -786,6 +795,7 @@ uint32_t vs_internal::wavefront_render(const vs::SceneView &view, const vs::Came
             launches += 4;
             // the any-hit rays run while the host takes the count
             hip_check(hipEventSynchronize(wb.ev_count), "wf sync");
+            if (stamps - read > 4u) read_stamps();
             queue.items = q[cur];
             queue.segment = segment;
             count = *wb.host_counts;
@@ -797,13 +807,7 @@ uint32_t vs_internal::wavefront_render(const vs::SceneView &view, const vs::Came
     }
     if (ts) {
         hip_check(hipStreamSynchronize(st), "wf sync");
-        for (size_t b = 0; b + 3 < stamps; b += 4)
-            for (int k = 0; k < 3; ++k) {
-                float ms = 0.f;
-                hip_check(hipEventElapsedTime(&ms, wb.ev[b + k], wb.ev[b + k + 1]), "event time");
-                ts->stage_ms[k] += ms;
-                ts->stage_launches[k] += 1;
-            }
+        if (stamps != read) read_stamps();
     }
     return launches;
 }

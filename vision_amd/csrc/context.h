@@ -99,14 +99,15 @@ struct WavefrontBuffers {
     DevBuf o, d, thr, L, meta, lam, lpdf, hit, sh_o, sh_d, sh_c, q0, q1, counts;
     uint32_t *host_counts{nullptr};// pinned
     hipEvent_t ev_count{nullptr};  // the live count is on the host
-    std::vector<hipEvent_t> ev;    // stage times, four a bounce, made as needed
+    hipEvent_t ev[8]{};            // stage times: four of a bounce, four of the next
     WavefrontBuffers() = default;
     WavefrontBuffers(const WavefrontBuffers &) = delete;
     WavefrontBuffers &operator=(const WavefrontBuffers &) = delete;
     ~WavefrontBuffers() {
         if (host_counts) (void)hipHostFree(host_counts);
         if (ev_count) (void)hipEventDestroy(ev_count);
-        for (hipEvent_t e : ev) (void)hipEventDestroy(e);
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
     }
 };
 
