@@ -57,3 +57,18 @@ def test_last_frame_without_accumulation(gpu_ctx):
     sc.render(3)
     assert np.array_equal(a.view(np.uint32), sc.film(0).view(np.uint32))
     sc.close()
+
+
+def test_depths_beyond_the_wavefronts_bounce_count(gpu_ctx, tmp_path):
+    """A scene file's max_depth has no limit; the wavefront's path state keeps
+    16 bits of the bounce, so deeper jobs stay with the megakernel."""
+    s = _scene("materials", tmp_path)
+    launches = []
+    for depth in (65_535, 65_536):
+        s["integrator"]["param"]["max_depth"] = depth
+        sc = gpu_ctx.load_text(s, str(tmp_path))
+        sc.build_accel()
+        sc.render(4)
+        launches.append(sc.stats()["launches"])
+        sc.close()
+    assert launches[0] > 1 and launches[1] == 1

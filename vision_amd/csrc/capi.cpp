@@ -845,7 +845,8 @@ constexpr uint32_t kWaveSpp = 3;
 bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, uint32_t &launches) {
     const uint64_t P = uint64_t(s->cam.width) * s->cam.height;
     if (!s->diffuse_only) {
-        if (spp < kWaveSpp) return false;
+        // the wavefront's path state keeps 16 bits of the bounce
+        if (spp < kWaveSpp || rv.max_depth > 0xFFFFu) return false;
         const uint32_t chunk = uint32_t(std::min<uint64_t>(spp, std::max<uint64_t>(1u, (32u << 20) / P)));
         if (P * chunk > 0xFFFFFFFFull || !wavefront_reserve(s->wf, size_t(P) * chunk)) return false;
         launches += wavefront_render(s->view, s->cam, rv, s->packed.rgb, false, s->film_rt.as<float4>(),
