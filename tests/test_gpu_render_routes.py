@@ -72,3 +72,31 @@ def test_depths_beyond_the_wavefronts_bounce_count(gpu_ctx, tmp_path):
         launches.append(sc.stats()["launches"])
         sc.close()
     assert launches[0] > 1 and launches[1] == 1
+
+
+@pytest.mark.parametrize("kind,spectral,depth,spp,size,routed", [
+    ("diffuse", 0, 2, 2, (1, 1), True), ("diffuse", 0, 2, 1, (64, 64), False),
+    ("diffuse", 0, 2, 2, (2048, 1024), True), ("diffuse", 0, 2, 2, (2048, 1025), False),
+    ("diffuse", 4, 2, 7, (1024, 512), True), ("diffuse", 4, 2, 7, (1024, 513), False),
+    ("diffuse", 4, 2, 8, (1024, 513), True), ("diffuse", 3, 2, 8, (2049, 1024), False),
+    ("materials", 0, 1, 3, (512, 512), True), ("materials", 0, 1, 3, (513, 512), False),
+    ("materials", 0, 2, 3, (1024, 512), True), ("materials", 4, 2, 3, (1025, 512), False),
+    ("materials", 0, 3, 3, (1024, 1024), True), ("materials", 0, 3, 8, (1025, 1024), False),
+    ("materials", 0, 4, 3, (2048, 1024), True), ("materials", 0, 4, 4, (2049, 1024), False),
+    ("materials", 0, 9, 3, (1024, 512), True), ("materials", 0, 9, 3, (1025, 512), False),
+    ("materials", 0, 8, 4, (2048, 2048), True), ("materials", 0, 8, 4, (2049, 2048), False),
+    ("materials", 0, 6, 2, (64, 64), False), ("materials", 0, 0, 3, (64, 64), False),
+])
+def test_routes(gpu_ctx, tmp_path, kind, spectral, depth, spp, size, routed):
+    """One launch is the megakernel; both sides of each line of the rule."""
+    sc = gpu_ctx.load_text(_scene(kind, tmp_path), str(tmp_path))
+    sc.build_accel()
+    sc.set_resolution(*size)
+    sc.set_integrator(depth, 5, 1.0)
+    if spectral:
+        sc.set_spectrum(True, spectral)
+    sc.render(spp)
+    launches = sc.stats()["launches"]
+    assert launches > 1 if routed else launches == 1
+    assert not routed or kind == "materials" or launches == 2
+    sc.close()

@@ -829,24 +829,59 @@ uint32_t render_wavefront(vs_scene *s, const vs::RenderView &rv0, uint32_t spp, 
 // samples in one lane (pt_kernel) would leave most of the GPU idle or wait on
 // diverging materials; the same film bit for bit.  False: not done here.
 //
-// Diffuse-family scenes: a lane a sample, up to 4 M pixels (the figures are at
-// pt_sample_kernel; above, the pixels alone fill the GPU many times over), in
-// chunks of up to 32 M samples (512 MB of radiance).
-// Every material: as wavefront, whose shading sorts paths by material, from
-// kWaveSpp samples a pixel on (up to 32 M paths at a time).  Its bounces are
-// launches with a host wait each, so one or two samples are done sooner by the
-// megakernel.  Measured (megakernel / wavefront ms, procedural scene of 80k
-// triangles, depth 16, sRGB) at 1, 2, 3, 4 and 8 samples: 96 x 54 1.3 / 2.1,
-// 2.5 / 2.4, 3.5 / 2.6, 4.7 / 2.7, 9.4 / 3.0; 639 x 361 1.7 / 3.4, 3.2 / 3.6,
-// 4.7 / 3.7, 6.1 / 3.8, 12.1 / 4.2; 1920 x 1080 2.7 / 4.3, 5.1 / 5.2, 7.3 /
-// 6.0, 9.8 / 6.9, 18.7 / 10.5; at depth 3 and with hero wavelengths alike.
+// Diffuse-family scenes: a lane a sample, in chunks of up to 32 M samples
+// (512 MB of radiance).  Every material: as wavefront, whose shading sorts paths
+// by material, up to 32 M paths at a time.
+//
+// Where the lines lie.  A lane a sample against a lane a pixel, times as much
+// the latter takes (Cornell box / 100k triangles, depth 8, 2 to 8 samples): at
+// 256 x 256 1.6 .. 2.6 / 1.6 .. 2.8, 512 x 512 1.09 .. 1.34 / 1.19 .. 1.52, full
+// HD 1.02 .. 1.05 / 1.07 .. 1.12, 2560 x 1440 0.98 .. 0.99 / 1.02 .. 1.04: the
+// pixels alone fill the GPU many times over.  With four hero wavelengths, whose
+// larger state spills more, 1.59 .. 2.2 / 1.56 .. 2.6, 0.95 .. 1.17 / 1.13 ..
+// 1.43, 1024 x 1024 0.95 .. 0.99 / 1.03 .. 1.08, full HD 0.96 .. 1.00 / 1.03 ..
+// 1.07, 2560 x 1440 0.93 .. 0.94 / 0.99 .. 1.00.
+constexpr uint64_t kSamplePixels = 1u << 21;
+constexpr uint64_t kSamplePixelsHero = 1u << 19;// fewer samples than kSampleSppHero
+constexpr uint32_t kSampleSppHero = 8;
+
+bool sample_lanes_pay(uint64_t pixels, uint32_t spp, bool hero) {
+    return pixels <= kSamplePixels && !(hero && pixels > kSamplePixelsHero && spp < kSampleSppHero);
+}
+
+// Wavefront against megakernel: the wavefront writes each path's state once
+// before the first bounce, so shallow jobs gain only while the megakernel's
+// waves are few; its bounces are launches with a host wait each, so one or two
+// samples, and few samples of deep paths, are done sooner by the megakernel.
+// Measured (what the megakernel takes, times, sRGB; one sphere under the sky /
+// four spheres / 16, 80k triangles / the Cornell box with glass and metal):
+//   depth 1  512 x 512, 3 samples  1.01 / 1.30 / 1.39 / 0.94
+//            1024 x 1024           0.78 / 0.78 / 0.83 / 0.74
+//   depth 2  724 x 724, 3          0.96 / 1.22 / 1.16 / 1.03
+//            full HD, 3            0.91 / 0.74 / 0.85 / 0.92
+//   depth 3  1024 x 1024, 3        1.03 / 1.07 / 1.03 / 1.03
+//            full HD, 3            1.03 / 0.88 / 0.99 / 1.03
+//   depth 4  full HD, 3            1.04 / 0.95 / 1.09 / 1.10
+//            2560 x 1440, 3        1.10 / 0.87 / 1.18 / 1.11
+//   depth 16 512 x 512, 3          0.97 / 1.38 / 1.49 / 1.31
+//            full HD, 3            0.78 / 1.23 / 1.31 / 1.54
+//            full HD, 4 and 8      0.86, 1.00 / 1.43, 1.98 / 1.51, 1.98 / 1.60, 1.70
+//            2560 x 1440, 4        0.97 / 1.25 / 1.40 / 1.62
+//            3840 x 2160, 4        1.07 / 1.00 / 1.36 / 1.57, mostly sky 0.84
 constexpr uint32_t kWaveSpp = 3;
+
+bool wavefront_pays(uint64_t pixels, uint32_t spp, uint32_t depth) {
+    // the wavefront's path state keeps 16 bits of the bounce
+    if (spp < kWaveSpp || depth == 0 || depth > 0xFFFFu) return false;
+    if (depth > 8 && spp < 4 && pixels > (1u << 19)) return false;
+    const uint32_t most = depth >= 8 && spp >= 4 ? 22u : 17u + std::min(depth, 4u);
+    return pixels <= (1ull << most);
+}
 
 bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, uint32_t &launches) {
     const uint64_t P = uint64_t(s->cam.width) * s->cam.height;
     if (!s->diffuse_only) {
-        // the wavefront's path state keeps 16 bits of the bounce
-        if (spp < kWaveSpp || rv.max_depth > 0xFFFFu) return false;
+        if (!wavefront_pays(P, spp, rv.max_depth)) return false;
         const uint32_t chunk = uint32_t(std::min<uint64_t>(spp, std::max<uint64_t>(1u, (32u << 20) / P)));
         if (P * chunk > 0xFFFFFFFFull || !wavefront_reserve(s->wf, size_t(P) * chunk)) return false;
         launches += wavefront_render(s->view, s->cam, rv, s->packed.rgb, false, s->film_rt.as<float4>(),
@@ -854,7 +889,7 @@ bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, uint32_t &laun
                                      nullptr, nullptr);
         return true;
     }
-    if (P > (4u << 20)) return false;
+    if (!sample_lanes_pay(P, spp, !s->packed.rgb)) return false;
     const uint32_t chunk = uint32_t(std::min<uint64_t>(std::min(spp, 65535u), (32u << 20) / P));
     if (s->samples.bytes < P * chunk * 16) {
         try {
