@@ -2,11 +2,14 @@
 way vs_render runs them (a lane a sample for the diffuse family, as wavefront
 for every material, one lane a pixel where counters or adaptive sampling need
 it), the film and the output buffer equal the frame-by-frame launches' bit for
-bit, also continued from an earlier frame, at odd sizes and without
-accumulation."""
+bit, also continued from an earlier frame, at odd sizes, in several chunks and
+without accumulation; and the workspace they run in is one of the context and
+given back."""
 import numpy as np
 import pytest
+import torch
 
+import vision_amd as va
 from vision_amd import scenegen
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +103,84 @@ def test_routes(gpu_ctx, tmp_path, kind, spectral, depth, spp, size, routed):
     assert launches > 1 if routed else launches == 1
     assert not routed or kind == "materials" or launches == 2
     sc.close()
+
+
+# a second chunk: of frames beyond a launch's grid, of samples beyond 32 M, and
+# of the wavefront's paths beyond 32 M
+@pytest.mark.parametrize("kind,size,spp,chunks", [("diffuse", (1, 1), 65_537, 2), ("diffuse", (1920, 1080), 17, 2),
+                                                  ("materials", (1920, 1080), 17, 2)])
+def test_jobs_of_several_chunks(gpu_ctx, tmp_path, kind, size, spp, chunks):
+    sc = gpu_ctx.load_text(_scene(kind, tmp_path), str(tmp_path))
+    sc.build_accel()
+    sc.set_resolution(*size)
+    sc.set_integrator(2 if kind == "diffuse" else 4, 5, 1.0)
+    sc.render(spp)
+    launches = sc.stats()["launches"]
+    # per chunk: samples and accumulation; or begin, accumulation and four launches a bounce, after one of the job
+    assert launches == 2 * chunks if kind == "diffuse" else launches >= 1 + chunks * (2 + 4 * 4)
+    got = sc.film(0)
+    sc.reset_film()
+    sc.set_counting(True)  # one launch of the megakernel
+    sc.render(spp)
+    assert sc.stats()["launches"] == 1
+    assert np.array_equal(sc.film(0).view(np.uint32), got.view(np.uint32))
+    sc.close()
+
+
+MB = 1 << 20
+
+
+def _free():
+    return torch.cuda.mem_get_info(0)[0]
+
+
+def _load(ctx, folder, kind="materials"):
+    sc = ctx.load_text(_scene(kind, folder), str(folder))
+    sc.build_accel()
+    sc.render(3)  # the kernels' code and scratch memory
+    sc.set_kernel("megakernel")
+    sc.set_resolution(256, 256)
+    return sc
+
+
+def test_scenes_share_a_workspace_that_is_given_back(tmp_path):
+    # 256 x 256 at 64 samples: 4 M paths, 772 MB of state, and 67 MB of samples
+    with va.Context(0) as ctx:
+        scenes = [_load(ctx, tmp_path) for _ in range(3)] + [_load(ctx, tmp_path, "diffuse")]
+        start = _free()
+        scenes[0].render(64)
+        one = start - _free()
+        assert 700 * MB < one < 900 * MB
+        for sc in scenes[1:]:
+            sc.render(64)
+            assert start - _free() < one + 100 * MB
+        scenes[1].set_kernel("megakernel")
+        assert start - _free() < 64 * MB
+        scenes[1].render(64)
+        assert start - _free() > 700 * MB
+        scenes.pop().close()
+        assert start - _free() < 64 * MB
+        for sc in scenes:
+            sc.close()
+
+
+def test_workspace_makes_room_for_other_allocations(tmp_path):
+    """A server's arena of more than is free beside the workspace (more than a
+    gigabyte beyond what the device reports can still be had)."""
+    with va.Context(0) as ctx:
+        sc = _load(ctx, tmp_path)
+        sc.render(256)  # 16 M paths, 3.1 GB
+        film = sc.film(0)
+        with va.Server(ctx, hbm_budget=_free() + 2500 * MB) as srv:
+            job = srv.submit(srv.add_scene(sc), 64, 64, 2)
+            srv.wait(job)
+            assert srv.result(job, 0, (64, 64)).max() > 0
+            # beside the arena, at most an eighth of what is free (and the pages of 14 buffers)
+            start = _free()
+            sc.reset_film()
+            sc.render(256)
+            held = -_free()
+            sc.set_kernel("megakernel")
+            assert held + _free() <= start // 8 + 32 * MB
+            assert np.array_equal(sc.film(0).view(np.uint32), film.view(np.uint32))
+        sc.close()

@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -307,6 +308,7 @@ vs_status vs_create(int32_t device, vs_context **out) {
     auto *ctx = new (std::nothrow) vs_context();
     if (!ctx) return VS_ERROR_OUT_OF_MEMORY;
     ctx->device = device;
+    ctx->work.device = device;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
         hipEventCreate(&ctx->tr0) != hipSuccess || hipEventCreate(&ctx->tr1) != hipSuccess ||
@@ -377,6 +379,7 @@ void vs_scene_destroy(vs_scene *scene) {
     if (scene->ctx && scene->ctx->device >= 0) {
         (void)hipSetDevice(scene->ctx->device);
         (void)hipStreamSynchronize(scene->ctx->stream);
+        (void)scene->ctx->work.give_back();
     }
     delete scene;
 }
@@ -389,6 +392,7 @@ vs_status vs_scene_set_kernel(vs_scene *s, int32_t mode, uint32_t chunk_frames, 
         return fail(s->ctx, VS_ERROR_INVALID_ARGUMENT, "chunk_frames must be in 1..1024");
     if (trace_block != 64 && trace_block != 128 && trace_block != 256)
         return fail(s->ctx, VS_ERROR_INVALID_ARGUMENT, "trace_block must be 64, 128 or 256");
+    (void)s->ctx->work.give_back();
     s->kernel_mode = uint32_t(mode);
     s->wf_chunk_frames = chunk_frames;
     s->wf_trace_block = trace_block;
@@ -693,6 +697,51 @@ namespace {
 
 }// extern "C"
 
+namespace {
+
+// the live contexts' workspaces
+struct Workspaces {
+    std::mutex mu;
+    std::vector<RenderWorkspace *> all;
+};
+Workspaces &workspaces() {
+    static Workspaces *w = new Workspaces();// contexts may outlive static objects
+    return *w;
+}
+
+}// namespace
+
+vs_internal::RenderWorkspace::RenderWorkspace() {
+    Workspaces &w = workspaces();
+    std::lock_guard<std::mutex> lk(w.mu);
+    w.all.push_back(this);
+}
+
+vs_internal::RenderWorkspace::~RenderWorkspace() {
+    Workspaces &w = workspaces();
+    std::lock_guard<std::mutex> lk(w.mu);
+    w.all.erase(std::find(w.all.begin(), w.all.end(), this));
+}
+
+bool vs_internal::RenderWorkspace::give_back() {
+    WorkspaceUse use(*this);
+    if (!use.mine || (!wf.capacity && !samples.ptr)) return false;
+    wf.release();
+    samples.release();
+    return true;
+}
+
+bool vs_internal::reclaim_workspaces() {
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess) return false;
+    Workspaces &w = workspaces();
+    std::lock_guard<std::mutex> lk(w.mu);
+    bool any = false;
+    for (RenderWorkspace *r : w.all)
+        if (r->device == device) any |= r->give_back();
+    return any;
+}
+
 bool vs_internal::wavefront_reserve(WavefrontBuffers &wb, size_t cap) {
     if (wb.capacity >= cap) return true;
     if (!wb.host_counts) {
@@ -701,19 +750,15 @@ bool vs_internal::wavefront_reserve(WavefrontBuffers &wb, size_t cap) {
         wb.host_counts = static_cast<uint32_t *>(hp);
     }
     if (!wb.ev_count) hip_check(hipEventCreateWithFlags(&wb.ev_count, hipEventDisableTiming), "event");
-    wb.capacity = 0;
-    DevBuf *all[] = {&wb.o, &wb.d, &wb.thr, &wb.L, &wb.meta, &wb.lam, &wb.lpdf, &wb.hit, &wb.sh_o, &wb.sh_d, &wb.sh_c,
-                     &wb.q0, &wb.q1, &wb.counts};
-    for (DevBuf *b : all) b->release();
+    wb.release();
     try {
         const size_t queue = vs::wf_queue_capacity(cap);
-        for (DevBuf *b : all) {
-            if (b == &wb.counts) b->alloc(vs::kWfWords * 4);
-            else if (b == &wb.q0 || b == &wb.q1) b->alloc(queue * 4);
-            else b->alloc((b == &wb.sh_o || b == &wb.sh_d || b == &wb.sh_c ? queue : cap) * 16);
-        }
+        for (DevBuf *b : {&wb.o, &wb.d, &wb.thr, &wb.L, &wb.meta, &wb.lam, &wb.lpdf, &wb.hit}) b->alloc(cap * 16);
+        for (DevBuf *b : {&wb.sh_o, &wb.sh_d, &wb.sh_c}) b->alloc(queue * 16);
+        for (DevBuf *b : {&wb.q0, &wb.q1}) b->alloc(queue * 4);
+        wb.counts.alloc(vs::kWfWords * 4);
     } catch (const DeviceError &) {
-        for (DevBuf *b : all) b->release();
+        wb.release();
         return false;
     }
     wb.capacity = cap;
@@ -878,33 +923,49 @@ bool wavefront_pays(uint64_t pixels, uint32_t spp, uint32_t depth) {
     return pixels <= (1ull << most);
 }
 
-bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, uint32_t &launches) {
+// paths or samples of a chunk, at most
+constexpr uint64_t kChunk = 32u << 20;
+
+// How many items of `bytes` a workspace that holds `held` may hold: an eighth of
+// the memory that is free without it.
+uint64_t workspace_items(uint64_t held, size_t bytes) {
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) return 0;
+    return (free + held * bytes) / 8 / bytes;
+}
+
+bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, RenderWorkspace &ws, uint32_t &launches) {
     const uint64_t P = uint64_t(s->cam.width) * s->cam.height;
-    if (!s->diffuse_only) {
-        if (!wavefront_pays(P, spp, rv.max_depth)) return false;
-        const uint32_t chunk = uint32_t(std::min<uint64_t>(spp, std::max<uint64_t>(1u, (32u << 20) / P)));
-        if (P * chunk > 0xFFFFFFFFull || !wavefront_reserve(s->wf, size_t(P) * chunk)) return false;
+    const bool wave = !s->diffuse_only;
+    if (wave ? !wavefront_pays(P, spp, rv.max_depth) : !sample_lanes_pay(P, spp, !s->packed.rgb)) return false;
+    const size_t bytes = wave ? WavefrontBuffers::kPathBytes : 16;
+    const uint64_t held = wave ? ws.wf.capacity : ws.samples.bytes / bytes;
+    uint64_t chunk = std::min<uint64_t>(wave ? spp : std::min(spp, 65535u), kChunk / P);
+    if (P * chunk > held) {
+        chunk = std::min(chunk, std::max(workspace_items(held, bytes), held) / P);
+        if (!chunk) return false;
+    }
+    if (wave) {
+        if (!wavefront_reserve(ws.wf, size_t(P) * chunk)) return false;
         launches += wavefront_render(s->view, s->cam, rv, s->packed.rgb, false, s->film_rt.as<float4>(),
-                                     s->film_out.as<float4>(), s->frame_index, spp, chunk, 64, s->wf, s->ctx->stream,
-                                     nullptr, nullptr);
+                                     s->film_out.as<float4>(), s->frame_index, spp, uint32_t(chunk), 64, ws.wf,
+                                     s->ctx->stream, nullptr, nullptr);
         return true;
     }
-    if (!sample_lanes_pay(P, spp, !s->packed.rgb)) return false;
-    const uint32_t chunk = uint32_t(std::min<uint64_t>(std::min(spp, 65535u), (32u << 20) / P));
-    if (s->samples.bytes < P * chunk * 16) {
+    if (P * chunk > held) {
         try {
-            s->samples.alloc(P * chunk * 16);
+            ws.samples.alloc(P * chunk * bytes);
         } catch (const DeviceError &) {
             return false;
         }
     }
     vs::WavefrontView w{};
-    w.L = s->samples.as<float4>();
+    w.L = ws.samples.as<float4>();
     w.pixels = uint32_t(P);
     w.width = s->cam.width;
-    for (uint32_t f = 0; f < spp; f += chunk) {
+    for (uint32_t f = 0; f < spp; f += uint32_t(chunk)) {
         rv.frame_start = s->frame_index + f;
-        rv.spp = std::min(chunk, spp - f);
+        rv.spp = std::min(uint32_t(chunk), spp - f);
         hip_check(vs::launch_pt_samples(s->view, s->cam, rv, w.L, s->ctx->stream), "pt samples");
         hip_check(vs::wf_accumulate(rv, w, rv.frame_start, rv.spp, s->film_rt.as<float4>(), s->film_out.as<float4>(),
                                     s->ctx->stream),
@@ -1211,6 +1272,7 @@ vs_status vs_render(vs_scene *s, uint32_t spp, int32_t fused) {
         }
         uint32_t launches = 0;
         vs_render_stats ts{};
+        const WorkspaceUse work(s->ctx->work);// until the job is through
         const bool restir = h.integrator.type == "rt";
         // adaptive sampling runs in the megakernel form (its statistics live
         // with the pixel's running mean)
@@ -1238,7 +1300,7 @@ vs_status vs_render(vs_scene *s, uint32_t spp, int32_t fused) {
             launches = render_restir(s, rv, spp, ctr, ts);
         } else if (wavefront) {
             launches = render_wavefront(s, rv, spp, ctr, ts);
-        } else if (fused && spp > 1 && !adaptive && !ctr && render_samples(s, rv, spp, launches)) {
+        } else if (fused && spp > 1 && !adaptive && !ctr && work.mine && render_samples(s, rv, spp, work.w, launches)) {
         } else if (fused) {
             rv.frame_start = s->frame_index;
             rv.spp = spp;

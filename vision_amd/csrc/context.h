@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -18,14 +19,6 @@
 #include "scene.h"
 #include "tables.h"
 
-struct vs_context {
-    int device{0};// -1: host-only context (scene parsing, BVH build, export)
-    hipStream_t stream{nullptr};
-    hipEvent_t ev0{nullptr}, ev1{nullptr};
-    hipEvent_t tr0{nullptr}, tr1{nullptr}, tr2{nullptr};// around wavefront traversal kernels
-    std::string last_error;
-};
-
 namespace vs_internal {
 
 struct DeviceError : std::runtime_error {
@@ -35,6 +28,10 @@ struct DeviceError : std::runtime_error {
 inline void hip_check(hipError_t e, const char *what) {
     if (e != hipSuccess) throw DeviceError(std::string(what) + ": " + hipGetErrorString(e));
 }
+
+// Gives back what idle contexts' workspaces hold on the current device; false
+// when that is nothing (capi.cpp)
+bool reclaim_workspaces();
 
 struct DevBuf {
     void *ptr{nullptr};
@@ -52,6 +49,10 @@ struct DevBuf {
         release();
         if (n == 0) n = 16;
         hipError_t e = hipMalloc(&ptr, n);
+        if (e != hipSuccess && reclaim_workspaces()) {
+            (void)hipGetLastError();
+            e = hipMalloc(&ptr, n);
+        }
         if (e != hipSuccess) {
             ptr = nullptr;
             (void)hipGetLastError();// the next launch does not report it again
@@ -102,6 +103,12 @@ struct WavefrontBuffers {
     hipEvent_t ev[8]{};            // stage times: four of a bounce, four of the next
     WavefrontBuffers() = default;
     WavefrontBuffers(const WavefrontBuffers &) = delete;
+    // bytes of path state and queues a path takes
+    static constexpr size_t kPathBytes = 11 * 16 + 2 * 4;
+    void release() {
+        capacity = 0;
+        for (DevBuf *b : {&o, &d, &thr, &L, &meta, &lam, &lpdf, &hit, &sh_o, &sh_d, &sh_c, &q0, &q1, &counts}) b->release();
+    }
     WavefrontBuffers &operator=(const WavefrontBuffers &) = delete;
     ~WavefrontBuffers() {
         if (host_counts) (void)hipHostFree(host_counts);
@@ -111,7 +118,47 @@ struct WavefrontBuffers {
     }
 };
 
+// What the megakernel form's jobs of several frames run in (render_samples):
+// path state of the wavefront, or single samples' radiance.  One of a context,
+// since one stream runs all its renders; at most 32 M paths and samples (6.2 and
+// 0.5 GB), and at the time of growing no more than an eighth of the device's free
+// memory.  Given back when an allocation of the library finds no room, when a
+// scene of the context goes, and by vs_scene_set_kernel.
+struct RenderWorkspace {
+    std::atomic<bool> busy{false};// a render uses it, or another thread gives it back
+    int device{-1};
+    WavefrontBuffers wf;
+    DevBuf samples;
+    RenderWorkspace();
+    ~RenderWorkspace();
+    RenderWorkspace(const RenderWorkspace &) = delete;
+    RenderWorkspace &operator=(const RenderWorkspace &) = delete;
+    // false when it is in use or held nothing
+    bool give_back();
+};
+
+// the workspace for the length of a call, if no other thread has it
+struct WorkspaceUse {
+    RenderWorkspace &w;
+    const bool mine;
+    explicit WorkspaceUse(RenderWorkspace &ws) : w(ws), mine(!ws.busy.exchange(true)) {}
+    ~WorkspaceUse() {
+        if (mine) w.busy = false;
+    }
+    WorkspaceUse(const WorkspaceUse &) = delete;
+    WorkspaceUse &operator=(const WorkspaceUse &) = delete;
+};
+
 }// namespace vs_internal
+
+struct vs_context {
+    int device{0};// -1: host-only context (scene parsing, BVH build, export)
+    hipStream_t stream{nullptr};
+    hipEvent_t ev0{nullptr}, ev1{nullptr};
+    hipEvent_t tr0{nullptr}, tr1{nullptr}, tr2{nullptr};// around wavefront traversal kernels
+    std::string last_error;
+    vs_internal::RenderWorkspace work;
+};
 
 using vs_internal::DevBuf;
 
@@ -134,7 +181,6 @@ struct vs_scene {
     bool diffuse_only{false};// only diffuse / Oren-Nayar / black materials
     DevBuf fis_lut, fis_cond, fis_cond_func, fis_marg, fis_marg_func;
     DevBuf film_rt, film_out, film_pic, counters;
-    DevBuf samples;// radiance of single camera samples (sample megakernel)
     DevBuf scratch_rays, scratch_hits;
     // wavefront form: per-path state, queues, append counters
     uint32_t kernel_mode{VS_KERNEL_MEGAKERNEL};
