@@ -39,18 +39,34 @@ def test_forward_of_a_list_equals_its_parts(cache, n):
     assert np.array_equal(whole.view(np.uint32), np.concatenate(parts).view(np.uint32))
 
 
-@pytest.mark.parametrize("n", [2, 17, 127, 129, 4099, 70001, (1 << 20) + 33])
-def test_gradients_are_the_mean_of_the_parts(cache, n):
+def _apart(whole, ref):
+    """The difference's norm in units of the tolerance: the gradients of three
+    layers are rounded to bf16 (2^-9 of each value), scaled by 1 / n in the whole
+    and by the parts' sizes in them, six roundings apart."""
+    whole, ref = np.asarray(whole, np.float64), np.asarray(ref, np.float64)
+    return np.linalg.norm(whole - ref) / (6 * 2.0 ** -9 * np.linalg.norm(ref))
+
+
+# the last `tail` rows (those of a second chunk of the workspace, or the very
+# last) have far larger targets, so that the sums are theirs.  They lie at one
+# point, where they have the same output and gradients in proportion to their
+# targets, and the last row has the largest: its share is 1 / 33 or more, 2.5
+# tolerances, and so a row lost, taken twice or at another's position shows
+@pytest.mark.parametrize("n,tail", [(2, 0), (17, 1), (127, 0), (129, 1), (4099, 0), (4099, 1), (70001, 0), (70001, 1),
+                                    ((1 << 20) + 33, 0), ((1 << 20) + 33, 33)])
+def test_gradients_are_the_mean_of_the_parts(cache, n, tail):
     rng = np.random.default_rng(n)
     s = np.concatenate([rng.uniform([-1, 0, -1], [1, 2, 1], (n, 3)), rng.exponential(0.5, (n, 3))], 1).astype(np.float32)
+    if tail:
+        s[-tail:, :3] = s[-1, :3]
+        s[-tail:, 3:] = 1e4 * rng.uniform(1, 2, (tail, 3))
+        s[-1, 3:] = 2e4
     cut = n // 2
-    loss, mlp, grid = cache.gradients(s)
-    (la, ma, ga), (lb, mb, gb) = cache.gradients(s[:cut]), cache.gradients(s[cut:])
-    wa, wb = cut / n, (n - cut) / n
-    for whole, a, b in ((loss, la, lb), (mlp, ma, mb), (grid, ga, gb)):
-        ref = wa * np.asarray(a, np.float64) + wb * np.asarray(b, np.float64)
-        # the gradients of three layers are rounded to bf16 (2^-9 of each
-        # value), scaled by 1 / n in the whole and by the parts' sizes in
-        # them: six roundings apart
-        tol = 6 * 2.0 ** -9 * np.linalg.norm(ref)
-        assert np.linalg.norm(np.asarray(whole, np.float64) - ref) <= tol
+    whole = cache.gradients(s)
+    a, b = cache.gradients(s[:cut]), cache.gradients(s[cut:])
+    for w, pa, pb in zip(whole, a, b):
+        assert _apart(w, cut / n * np.asarray(pa, np.float64) + (n - cut) / n * np.asarray(pb, np.float64)) <= 1
+    if tail:
+        fewer = cache.gradients(s[:-1])
+        for w, p in zip(whole, fewer):
+            assert _apart(w, (n - 1) / n * np.asarray(p, np.float64)) > 2
