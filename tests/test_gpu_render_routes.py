@@ -79,9 +79,8 @@ def test_depths_beyond_the_wavefronts_bounce_count(gpu_ctx, tmp_path):
 
 @pytest.mark.parametrize("kind,spectral,depth,spp,size,routed", [
     ("diffuse", 0, 2, 2, (1, 1), True), ("diffuse", 0, 2, 1, (64, 64), False),
-    ("diffuse", 0, 2, 2, (2048, 1024), True), ("diffuse", 0, 2, 2, (2048, 1025), False),
-    ("diffuse", 4, 2, 7, (1024, 512), True), ("diffuse", 4, 2, 7, (1024, 513), False),
-    ("diffuse", 4, 2, 8, (1024, 513), True), ("diffuse", 3, 2, 8, (2049, 1024), False),
+    ("diffuse", 0, 2, 2, (2048, 2048), True), ("diffuse", 0, 2, 2, (2048, 2049), False),
+    ("diffuse", 4, 2, 2, (2048, 2048), True), ("diffuse", 3, 2, 3, (2049, 2048), False),
     ("materials", 0, 1, 3, (512, 512), True), ("materials", 0, 1, 3, (513, 512), False),
     ("materials", 0, 2, 3, (1024, 512), True), ("materials", 4, 2, 3, (1025, 512), False),
     ("materials", 0, 3, 3, (1024, 1024), True), ("materials", 0, 3, 8, (1025, 1024), False),

@@ -879,20 +879,13 @@ uint32_t render_wavefront(vs_scene *s, const vs::RenderView &rv0, uint32_t spp, 
 // by material, up to 32 M paths at a time.
 //
 // Where the lines lie.  A lane a sample against a lane a pixel, times as much
-// the latter takes (Cornell box / 100k triangles, depth 8, 2 to 8 samples): at
-// 256 x 256 1.6 .. 2.6 / 1.6 .. 2.8, 512 x 512 1.09 .. 1.34 / 1.19 .. 1.52, full
-// HD 1.02 .. 1.05 / 1.07 .. 1.12, 2560 x 1440 0.98 .. 0.99 / 1.02 .. 1.04: the
-// pixels alone fill the GPU many times over.  With four hero wavelengths, whose
-// larger state spills more, 1.59 .. 2.2 / 1.56 .. 2.6, 0.95 .. 1.17 / 1.13 ..
-// 1.43, 1024 x 1024 0.95 .. 0.99 / 1.03 .. 1.08, full HD 0.96 .. 1.00 / 1.03 ..
-// 1.07, 2560 x 1440 0.93 .. 0.94 / 0.99 .. 1.00.
-constexpr uint64_t kSamplePixels = 1u << 21;
-constexpr uint64_t kSamplePixelsHero = 1u << 19;// fewer samples than kSampleSppHero
-constexpr uint32_t kSampleSppHero = 8;
-
-bool sample_lanes_pay(uint64_t pixels, uint32_t spp, bool hero) {
-    return pixels <= kSamplePixels && !(hero && pixels > kSamplePixelsHero && spp < kSampleSppHero);
-}
+// the latter takes (Cornell box / 100k triangles / a closed furnace, depth 8, 2
+// and 8 samples): at 256 x 256 1.64, 2.78 / 1.68, 2.90 / 1.61, 2.52, 512 x 512
+// 1.17, 1.41 / 1.20, 1.50 / 1.11, 1.30, full HD 1.08, 1.14 / 1.06, 1.11 / 1.06,
+// 1.07, 2048 x 2048 1.02 / 0.99 / 1.05: the pixels alone fill the GPU many times
+// over.  With hero wavelengths 1.92, 2.97 / 1.84, 3.01 / 1.99, 3.01 .. 2048 x 2048
+// 1.19 / 1.05 / 1.37.
+constexpr uint64_t kSamplePixels = 1u << 22;
 
 // Wavefront against megakernel: the wavefront writes each path's state once
 // before the first bounce, so shallow jobs gain only while the megakernel's
@@ -937,7 +930,7 @@ uint64_t workspace_items(uint64_t held, size_t bytes) {
 bool render_samples(vs_scene *s, vs::RenderView rv, uint32_t spp, RenderWorkspace &ws, uint32_t &launches) {
     const uint64_t P = uint64_t(s->cam.width) * s->cam.height;
     const bool wave = !s->diffuse_only;
-    if (wave ? !wavefront_pays(P, spp, rv.max_depth) : !sample_lanes_pay(P, spp, !s->packed.rgb)) return false;
+    if (wave ? !wavefront_pays(P, spp, rv.max_depth) : P > kSamplePixels) return false;
     const size_t bytes = wave ? WavefrontBuffers::kPathBytes : 16;
     const uint64_t held = wave ? ws.wf.capacity : ws.samples.bytes / bytes;
     uint64_t chunk = std::min<uint64_t>(wave ? spp : std::min(spp, 65535u), kChunk / P);

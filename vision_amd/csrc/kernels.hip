@@ -82,13 +82,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MS == M
 // L[frame * pixels + pixel] for the film to fold in frame order.  A pixel's
 // samples in one lane (pt_kernel) leave the chip to width * height / 64 waves,
 // one a SIMD for a 256 x 256 job, each as long as its slowest lane's samples
-// together.  Measured against pt_kernel, diffuse family: Cornell box 256 x 256
-// 16 spp 2.76 -> 0.86 ms, 64 x 48 64 spp 9.6 -> 0.27 ms, 100k triangles 512 x
-// 512 16 spp hero-4 10.96 -> 6.89 ms, 1920 x 1080 4 spp 8.79 -> 8.24 ms (2 to 4
-// samples a lane: 7.77 and 7.17 ms on the third; 16 or 32 pixels a wave were
-// slower throughout).
+// together.  2 to 4 samples a lane, and 16 or 32 pixels a wave, were slower.
+// Bound by the latency of the traversal and by divergence, and by what the
+// register budget spills: at 4, 5 and 6 waves a SIMD the Cornell box of 1920 x
+// 1080, 16 samples, depth 8 takes 12.29, 12.28 and 13.07 ms, a closed furnace
+// (8 samples) 7.2, 7.3 and 8.6, 100k triangles 23.8, 23.3 and 22.9; with four
+// hero wavelengths the box takes 15.4, 19.8 and 19.9, 100k triangles 27.2, 30.4
+// and 29.4.  With the six waves of pt_kernel large jobs were slower than there.
 template <int NS, bool RGB>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RGB ? 5 : 4)))
 pt_sample_kernel(SceneView sc, CameraView cam, RenderView rv, float4 *__restrict__ L) {
     extern __shared__ uint2 lds_stack[];
     const uint32_t px = blockIdx.x * 8u + (threadIdx.x & 7u);
