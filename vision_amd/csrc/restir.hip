@@ -35,16 +35,20 @@ __device__ __forceinline__ void add_counters(unsigned long long *counters, const
     atomicAdd(counters + 2, (unsigned long long)pc.tris);
 }
 
-// Register budget of shader0 and shader1: four resident waves per SIMD for
-// the diffuse family (128 VGPRs; the compiler alone takes 161-187 and
-// three or two waves).  Measured on the 1080p many-lights job (64 frames):
-// shader0 150.7 -> 139.6 ms, shader1 59.9 -> 54.2 ms; five and six waves
-// were slower, and the spatial pass is fastest left free.  Kernels for
-// every material keep the compiler's choice (not measured).
-constexpr int restir_waves(int ms) { return ms == MS_ALL ? 1 : 4; }
+// Register budgets of shader0 and shader1 for the diffuse family, in resident
+// waves per SIMD: three and four (168 and 128 VGPRs; the compiler alone takes
+// 161-187 and three or two waves).  Shader0 spills 130 registers at four, since
+// the traversal's byte selectors are live through it: whole frames of the Cornell
+// box at 1280 x 720 take 0.39, 0.34, 0.39 and 0.50 ms at 2, 3, 4 and 5 waves (0.37
+// before the selectors), of 4000 emitters at 1920 x 1080 1.78, 1.53, 1.53 and 1.68.
+// Shader1: 59.9 -> 54.2 ms of the 1080p many-lights job (64 frames); five and six
+// waves were slower, and the spatial pass is fastest left free.  Kernels for every
+// material keep the compiler's choice (not measured).
+constexpr int initial_waves(int ms) { return ms == MS_ALL ? 1 : 3; }
+constexpr int final_waves(int ms) { return ms == MS_ALL ? 1 : 4; }
 
 template <int NS, bool RGB, int MS>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(restir_waves(MS)))) initial_kernel(SceneView sc, CameraView cam, RestirView v,
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(initial_waves(MS)))) initial_kernel(SceneView sc, CameraView cam, RestirView v,
                                                      unsigned long long *__restrict__ counters) {
     extern __shared__ uint2 lds_stack[];
     const uint2 tile = xcd_tile_2d();
@@ -69,7 +73,7 @@ __global__ void __launch_bounds__(64) spatial_kernel(SceneView sc, RestirView v,
 // shader1 plus the film's running mean (RealTimeIntegrator's combine,
 // rt.cpp:121-130, with the indirect half absent)
 template <int NS, bool RGB, int MS>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(restir_waves(MS)))) final_kernel(SceneView sc, CameraView cam, RestirView v, RenderView rv,
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(final_waves(MS)))) final_kernel(SceneView sc, CameraView cam, RestirView v, RenderView rv,
                                                    uint32_t in, float4 *__restrict__ rt, float4 *__restrict__ out,
                                                    unsigned long long *__restrict__ counters) {
     extern __shared__ uint2 lds_stack[];
