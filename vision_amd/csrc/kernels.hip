@@ -53,15 +53,17 @@ __global__ void __launch_bounds__(256) trace_kernel(SceneView sc, const RayRec *
 // carried per path; RGB: sRGB mode (three fixed channels) vs hero wavelengths.
 // The kernel asks for a number of resident waves per SIMD that spills some
 // state to scratch: traversal latency is better hidden by more waves than
-// lost to the spills.  Measured on one MI355X: the diffuse family at six
-// waves (80 VGPRs; 1.25-1.55x over the compiler's own choice on diffuse
-// scenes, four waves 5 % slower); every material at four (128 VGPRs; 6 waves:
-// 466 ms, 5: 441 ms, 4: 428 ms, 3: 473 ms for the procedural 1080p
-// 64-spp hero-4 job).
+// lost to the spills.  Measured on one MI355X: the diffuse family in sRGB at
+// six waves (80 VGPRs; 1.25-1.55x over the compiler's own choice on diffuse
+// scenes), with hero wavelengths at four (one sample a pixel, full HD, depth 8:
+// a closed furnace 1.95 ms at six, 1.61 at five, 1.57 at four, the Cornell box
+// 1.31, 1.19, 1.16, 100k triangles 2.06, 2.01, 2.01); every material at four
+// (128 VGPRs; 6 waves: 466 ms, 5: 441 ms, 4: 428 ms, 3: 473 ms for the
+// procedural 1080p 64-spp hero-4 job).
 // ADAPT: adaptive sampling on (rv.vstats holds the per-pixel statistics).
 // COUNT: rays and BVH fetches tallied into counters.
 template <int NS, bool RGB, int MS, bool ADAPT, bool COUNT>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MS == MS_ALL ? 4 : 6))) pt_kernel(SceneView sc, CameraView cam, RenderView rv,
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MS == MS_ALL || !RGB ? 4 : 6))) pt_kernel(SceneView sc, CameraView cam, RenderView rv,
                                                   float4 *__restrict__ rt, float4 *__restrict__ out,
                                                   unsigned long long *__restrict__ counters) {
     extern __shared__ uint2 lds_stack[];
