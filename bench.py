@@ -26,7 +26,10 @@ run of the same job divided by that kernel's event time.  Traversal bytes
 per ray: BVH8 node fetches x 80 B + leaf-triangle fetches x 48 B + 48 B ray
 in / hit out.  Per-unit record bytes (the records the kernel reads and
 writes, cache hits included):
-  megakernel PT: traversal + 32 B film read / write per pixel;
+  megakernel PT (the stats' launches tell how vs_render ran the job): one
+      launch: traversal + 32 B film read / write per pixel; a lane a sample:
+      as much + 32 B radiance written and read per sample; as wavefront: all
+      its stages below + 176 B of state written and 16 B read per sample;
   persistent serving kernel: traversal + 32 B film per sample (the first
       --count-jobs jobs, routed as in the timed run, are run once timed and
       once counting; jobs of --lane-min-samples samples or more go to the
@@ -34,9 +37,11 @@ writes, cache hits included):
       kernel is the one of the persistent kernel and the three lane stages
       with the most event time);
   wavefront closest-hit: traversal;
-  wavefront shading: SHADE_BYTES per shaded path (path state 96 in,
-      64 + 32 out, hit, queues, triangle, vertices, instance, material, light)
-      + 48 B per shadow ray written;
+  wavefront shading: SHADE_BYTES per shaded path (path state in, hit, queue,
+      triangle, vertices, instance, material, light; 32 B more of wavelengths
+      with hero wavelengths) + 68 B per path that goes on (state and queue out)
+      + 48 B per shadow ray written; left out, since not counted: 32 B of each
+      path whose bounce adds radiance;
   wavefront any-hit: traversal + 32 B per shadow ray (contribution, radiance);
   ReSTIR shader0: traversal + 4 x 48 B records (surface and reservoir
       written, previous frame's read) + 124 B surface gathers + 128 B
@@ -67,7 +72,15 @@ RECORD_BYTES = 48      # ReSTIR surface / reservoir record
 SURFACE_GATHER = 124   # triangle indices 12 + positions 36 + normals 36 + uvs 24 + instance 16
 MATERIAL_BYTES = 128
 CANDIDATE_BYTES = 184  # light selection alias 8 + func 4, light record 112, triangle alias 12, triangle 48
-SHADE_BYTES = 192 + 16 + 8 + SURFACE_GATHER + MATERIAL_BYTES + CANDIDATE_BYTES
+SHADE_BYTES = 64 + 16 + 4 + SURFACE_GATHER + MATERIAL_BYTES + CANDIDATE_BYTES
+HERO_BYTES = 32        # wavelengths and their pdfs
+
+
+def shade_bytes(shaded: int, samples: int, shadow_rays: int, hero: bool) -> int:
+    """What the wavefront's shading reads and writes for `shaded` paths of
+    `samples` camera samples (all but a path's first shading follow one that
+    let it go on)."""
+    return ((SHADE_BYTES + HERO_BYTES * hero) * shaded + (64 + 4) * (shaded - samples) + RAY_BYTES * shadow_rays)
 
 
 SCENE_CACHE = ROOT / "vision_amd" / "_scenes"
@@ -207,8 +220,8 @@ def serve_jobs(n: int, n_scenes: int, seed: int = 0) -> list:
 
 def plain_job(sc, job: dict) -> float:
     """One job the plain way: switch the scene to the job's spectrum mode,
-    resolution and depth, render all its frames in one megakernel launch,
-    download the output film.  Returns its service time in seconds."""
+    resolution and depth, render all its frames in one call of the megakernel
+    form, download the output film.  Returns its service time in seconds."""
     t0 = time.perf_counter()
     sc.set_spectrum(job["spectral"], 4)
     sc.set_resolution(job["width"], job["height"])
@@ -399,7 +412,8 @@ def serve_main(args) -> None:
         k = stage_names.index(kernel)
         trav = lambda t: (NODE_BYTES * st_cnt["lane_node_fetches"][t] + TRI_BYTES * st_cnt["lane_tri_fetches"][t] +
                           RAY_BYTES * st_cnt["lane_rays"][t])
-        alg_bytes = [trav(0), SHADE_BYTES * st_cnt["lane_rays"][0] + RAY_BYTES * st_cnt["lane_rays"][1],
+        # the lanes' sRGB and hero jobs are not counted apart: without the wavelengths
+        alg_bytes = [trav(0), shade_bytes(st_cnt["lane_rays"][0], lane_samples, st_cnt["lane_rays"][1], False),
                      trav(1) + 32 * st_cnt["lane_rays"][1]][k]
         unit_samples, launches = lane_samples, st_time["lane_stage_launches"][k]
         tr = measured_traffic(kernel.split()[0] + "@serving_mix_lanes")
@@ -869,14 +883,21 @@ def plain_workload(name: str, steps: int, warmup: int, kernel_form: str, chunk_f
     samples = W * H * spp
     msps = samples * steps / wall / 1e6
 
-    # counting run of the same job: rays, node and triangle fetches
+    # counting run of the same job: rays, node and triangle fetches.  Counted
+    # megakernel jobs are one launch whatever way the timed ones ran, so a job
+    # that ran as wavefront (more launches than a chunk's two) is counted so
+    staged = restir or kernel_form == "wavefront"
+    launches = stats[0]["launches"]
+    diffuse = name == "cbox"
+    as_wave = not staged and launches > 1 and not diffuse
+    if as_wave:
+        sc.set_kernel("wavefront", max(1, min(1024, spp, (32 << 20) // (W * H))), 64)
     sc.set_counting(True)
     cst = step()
     sc.set_counting(False)
     trav = lambda k: (NODE_BYTES * cst["stage_node_fetches"][k] + TRI_BYTES * cst["stage_tri_fetches"][k] +
                       RAY_BYTES * cst["stage_rays"][k])
     avg_kernel_s = sum(s["kernel_ms"] for s in stats) / len(stats) / 1e3
-    staged = restir or kernel_form == "wavefront"
     if staged:
         stage_s = [sum(s["stage_ms"][k] for s in stats) / len(stats) / 1e3 for k in range(3)]
         k = max(range(3), key=lambda i: stage_s[i])
@@ -894,7 +915,8 @@ def plain_workload(name: str, steps: int, warmup: int, kernel_form: str, chunk_f
             names = ["trace_queue_kernel (wavefront closest-hit traversal)", "shade_kernel (wavefront shading)",
                      "shadow_kernel (wavefront any-hit traversal)"]
             if k == 1:
-                alg_bytes = SHADE_BYTES * cst["stage_rays"][0] + RAY_BYTES * cst["stage_rays"][2]
+                alg_bytes = shade_bytes(cst["stage_rays"][0], samples, cst["stage_rays"][2],
+                                        config["spectrum"] != "srgb")
             elif k == 0:
                 alg_bytes = trav(0)
             else:
@@ -902,14 +924,21 @@ def plain_workload(name: str, steps: int, warmup: int, kernel_form: str, chunk_f
         kernel, kernel_s, launches = names[k], stage_s[k], cst["stage_launches"][k]
     else:
         kernel_s = avg_kernel_s
-        launches = cst["launches"]
         alg_bytes = (NODE_BYTES * cst["node_fetches"] + TRI_BYTES * cst["tri_fetches"] + RAY_BYTES * cst["rays"] +
                      FILM_BYTES * W * H)
-        kernel = "pt_kernel (megakernel)"
+        if launches == 1:
+            kernel = "pt_kernel (megakernel)"
+        elif diffuse:
+            alg_bytes += 32 * samples
+            kernel = "pt_sample_kernel + accumulate_kernel (megakernel form, a lane a sample)"
+        else:
+            alg_bytes += ((176 + 16) * samples + 32 * cst["stage_rays"][2] +
+                          shade_bytes(cst["stage_rays"][0], samples, cst["stage_rays"][2], config["spectrum"] != "srgb"))
+            kernel = "wavefront kernels (megakernel form, every material)"
     achieved = alg_bytes / kernel_s / 1e9
     mrays = cst["rays"] / avg_kernel_s / 1e6
     tag = {"procedural": "procedural_1080p_64spp_hero4", "restir": "restir_many_lights_1080p_64frames"}.get(name)
-    tr = measured_traffic(kernel.split()[0] + "@" + tag) if tag else None
+    tr = measured_traffic(kernel.split()[0] + "@" + tag) if tag and (staged or launches == 1) else None
     if tr and staged and not restir and (tr.get("chunk_frames"), tr.get("trace_block")) != (chunk_frames, trace_block):
         tr = None  # measured at another launch shape: bytes per launch differ
     film = sc.film(0)
