@@ -226,7 +226,11 @@ vs_status vs_scene_bsdf(vs_scene *scene, uint32_t mat, uint32_t n, const float *
 
 /* Kernel form of vs_render.  MEGAKERNEL: a thread runs whole paths (fused or
  * per-frame launches; a fused job of several frames may run its samples in
- * threads of their own, or as wavefront, where that is faster).  WAVEFRONT: the bounce loop split into
+ * threads of their own, or as wavefront, where that is faster, in a workspace
+ * that the context's scenes share: up to 6.7 GB, and no more than an eighth of
+ * the device memory that is free when it grows.  It is given back when an
+ * allocation of this library finds no room, when a scene of the context is
+ * destroyed, and by this call).  WAVEFRONT: the bounce loop split into
  * closest-hit / shade / any-hit kernels over queues of live paths held in
  * HBM, `chunk_frames` frames of all pixels per chunk, traversal blocks of
  * `trace_block` (64, 128 or 256) threads.  Both give the same film.  No
@@ -239,8 +243,9 @@ vs_status vs_scene_set_kernel(vs_scene *scene, int32_t mode, uint32_t chunk_fram
 /* Add `spp` progressive frames to the film (frame indices continue from the
  * current one).  fused = 0: one launch per frame, as
  * PathTracingIntegrator::render does (src/render_core/integrators/pt.cpp:90-99);
- * fused = 1: one launch adding all frames with the running mean in registers.
- * Both produce the same film.  With the "rt" integrator each frame runs ReSTIR
+ * fused = 1: all frames together, as one launch with the running mean in
+ * registers or in the forms described at vs_scene_set_kernel (the stats'
+ * launches tell).  Both produce the same film.  With the "rt" integrator each frame runs ReSTIR
  * DI (RealTimeIntegrator::render, src/render_core/integrators/rt.cpp:144-160,
  * direct half): initial candidates + temporal reuse, any extra spatial
  * passes, spatial reuse + shading; with the "indirect" block open (sRGB

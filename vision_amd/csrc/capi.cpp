@@ -880,11 +880,11 @@ uint32_t render_wavefront(vs_scene *s, const vs::RenderView &rv0, uint32_t spp, 
 //
 // Where the lines lie.  A lane a sample against a lane a pixel, times as much
 // the latter takes (Cornell box / 100k triangles / a closed furnace, depth 8, 2
-// and 8 samples): at 256 x 256 1.64, 2.78 / 1.68, 2.90 / 1.61, 2.52, 512 x 512
-// 1.17, 1.41 / 1.20, 1.50 / 1.11, 1.30, full HD 1.08, 1.14 / 1.06, 1.11 / 1.06,
-// 1.07, 2048 x 2048 1.02 / 0.99 / 1.05: the pixels alone fill the GPU many times
-// over.  With hero wavelengths 1.92, 2.97 / 1.84, 3.01 / 1.99, 3.01 .. 2048 x 2048
-// 1.19 / 1.05 / 1.37.
+// and 8 samples): at 256 x 256 1.62, 2.76 / 1.67, 2.91 / 1.61, 2.51, 512 x 512
+// 1.17, 1.41 / 1.19, 1.50 / 1.11, 1.30, full HD 1.08, 1.11 / 1.06, 1.12 / 1.06,
+// 1.07, 2048 x 2048 1.02 / 1.00 / 1.04: the pixels alone fill the GPU many times
+// over.  With four hero wavelengths 1.66, 2.53 / 1.65, 2.74 / 1.54, 2.26, full HD
+// 1.10, 1.15 / 1.08, 1.12 / 1.13, 1.14, 2048 x 2048 1.07 / 1.05 / 1.11.
 constexpr uint64_t kSamplePixels = 1u << 22;
 
 // Wavefront against megakernel: the wavefront writes each path's state once

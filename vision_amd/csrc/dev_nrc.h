@@ -1,8 +1,9 @@
 // Device code of the radiance cache: hash-grid encoding, the MLP on BF16
 // MFMA tiles (16x16x16, FP32 accumulation) and its backward pass.
 //
-// A wave takes 64 rows (queries) or 32 (training samples), encodes them and
-// sends them through the network in tiles of 16.  Tile operands live in LDS:
+// The encoding is a kernel of its own.  A wave of the network's kernels takes 64
+// encoded rows (queries) or 16 (training samples) at a time and sends them
+// through the network in tiles of 16.  Tile operands live in LDS:
 // activations row-major (bf16), weights transposed (wt[n][k] = W[k][n]) and,
 // for the backward pass, also as they are, so that a lane's four consecutive k
 // of an MFMA operand are one 8-byte load.  MFMA lane layout (16x16x16 bf16):

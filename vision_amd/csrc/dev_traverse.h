@@ -2,8 +2,9 @@
 // OptiX Accel::trace_closest / trace_occlusion, src/base/mgr/geometry.cpp:167-184).
 //
 // Per lane: one stack of node groups in LDS (entry = child_base, remaining
-// hit bits in near-to-far visiting order, internal-child mask), at most one
-// entry per tree level.  Leaf triangles of a node are tested before the next
+// hit bits by slot, internal-child mask), at most one entry per tree level; the
+// nearest slot is picked by the ray's octant when a child is fetched
+// (first_slot).  Leaf triangles of a node are tested before the next
 // node is fetched, so closest-hit culling uses the tightest t.
 //
 // The ray/triangle test is the watertight test of Woop, Benthin and Wald

@@ -599,7 +599,12 @@ namespace {
 
 // features of rows [first, first + span), sixteen rows a lane from half a
 // million on: 1 M rows took 437 us at one row a lane, 381 at four, 344 at eight
-// and 270 at sixteen (a wave a SIMD), 65536 rows 29 us at one
+// and 270 at sixteen (a wave a SIMD), 65536 rows 29 us at one.  Whole lookups from
+// host arrays, at one / eight / sixteen rows: 65536 136 / 277 / 449 us, 200 k 422 /
+// 447 / 584, 262144 491 / 503 / 624, 350 k 684 / 656 / 737, 460 k 853 / 765 / 851,
+// 524288 937 / 849 / 921, 600 k 1055 / 1142 / 991, 800 k 1434 / 1400 / 1294: one
+// and sixteen cross below half a million, and eight rows, not built, would be up
+// to a tenth of the call faster from 350 to 530 k.
 hipError_t encode(const NrcView &v, const float *pos, uint32_t stride, const uint32_t *count, uint32_t cap,
                   uint32_t offset, uint32_t batch, uint32_t first, uint32_t span, uint32_t *feat, hipStream_t s) {
     if (span >= (1u << 19))

@@ -103,12 +103,14 @@ __global__ void __launch_bounds__(256) begin_kernel(CameraView cam, RenderView r
     store_begin<NS, RGB>(w, i, ps);
 }
 
-// The traversal kernels at seven waves per SIMD (72 VGPRs): the procedural
-// 1080p 64-spp hero-4 job traces in 59.3 / 36.5 ms (closest / any hit), at six
-// waves 59.4 / 36.9, at eight (which spill) 60.1 / 39.6; with byte-to-float
-// conversions and selects in the slab tests they took 70.2 / 40.8.  Waves that
-// own 512 rays of the queue and refill their finished lanes were no faster
-// (62.1 / 38.2): a node's triangles, not the rays' lengths, leave lanes idle.
+// The traversal kernels at seven waves per SIMD (72 VGPRs): the 1080p 64-spp
+// hero-4 job of 320k triangles traces in 61.7 / 38.0 ms (closest / any hit), with
+// byte-to-float conversions and selects in the slab tests in 70.3 / 40.8.  The
+// budgets were compared on a node with tighter boxes (6 % fewer visits): 59.3 /
+// 36.5 at seven waves, 59.4 / 36.9 at six, 60.1 / 39.6 at eight, which spill; and
+// waves that own 512 rays of the queue and refill their finished lanes were no
+// faster there (62.1 / 38.2): a node's triangles, not the rays' lengths, leave
+// lanes idle.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 trace_queue_kernel(SceneView sc, WavefrontView w, WavefrontQueue queue, uint32_t count,
                    unsigned long long *__restrict__ counters) {
