@@ -183,3 +183,29 @@ def test_workspace_makes_room_for_other_allocations(tmp_path):
             assert held + _free() <= start // 8 + 32 * MB
             assert np.array_equal(sc.film(0).view(np.uint32), film.view(np.uint32))
         sc.close()
+
+
+def test_workspace_makes_room_for_another_scenes_render(tmp_path):
+    """A wavefront job that needs 7.6 GB of state where 2.5 GB are free beside
+    the workspace's 6.1."""
+    with va.Context(0) as ctx:
+        a, b = _load(ctx, tmp_path), _load(ctx, tmp_path)
+        for sc in (a, b):
+            sc.set_resolution(1920, 1080)
+            sc.set_integrator(2, 5, 1.0)
+        b.set_kernel("wavefront", chunk_frames=1)
+        b.render(1)
+        b.set_kernel("wavefront", chunk_frames=20)
+        a.set_integrator(4, 5, 1.0)
+        a.render(16)
+        rest = torch.empty(_free() - 2500 * MB, dtype=torch.uint8, device="cuda")
+        b.reset_film()
+        b.render(20)
+        film = b.film(0)
+        del rest
+        torch.cuda.empty_cache()
+        b.reset_film()
+        b.render(20, fused=False)
+        assert np.array_equal(b.film(0).view(np.uint32), film.view(np.uint32))
+        b.close()
+        a.close()

@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <optional>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -1265,13 +1266,16 @@ vs_status vs_render(vs_scene *s, uint32_t spp, int32_t fused) {
         }
         uint32_t launches = 0;
         vs_render_stats ts{};
-        const WorkspaceUse work(s->ctx->work);// until the job is through
         const bool restir = h.integrator.type == "rt";
         // adaptive sampling runs in the megakernel form (its statistics live
         // with the pixel's running mean)
         const bool adaptive = !restir && h.integrator.adaptive.on;
         const bool wavefront = !restir && !adaptive && s->kernel_mode == VS_KERNEL_WAVEFRONT;
         const bool staged = restir || wavefront;// two counter sets, [0..2] and [4..6]
+        // taken until the job is through, and by no other job: what those
+        // allocate may need it given back
+        std::optional<WorkspaceUse> work;
+        if (fused && spp > 1 && !staged && !adaptive && !ctr) work.emplace(s->ctx->work);
         if (!restir) {
             // ConvergenceInspector::reset at frame 0 (pt.cpp:93-95)
             const uint32_t P = s->cam.width * s->cam.height;
@@ -1293,7 +1297,7 @@ vs_status vs_render(vs_scene *s, uint32_t spp, int32_t fused) {
             launches = render_restir(s, rv, spp, ctr, ts);
         } else if (wavefront) {
             launches = render_wavefront(s, rv, spp, ctr, ts);
-        } else if (fused && spp > 1 && !adaptive && !ctr && work.mine && render_samples(s, rv, spp, work.w, launches)) {
+        } else if (work && work->mine && render_samples(s, rv, spp, work->w, launches)) {
         } else if (fused) {
             rv.frame_start = s->frame_index;
             rv.spp = spp;
