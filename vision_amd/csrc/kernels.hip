@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MS == M
 // 1080, 16 samples, depth 8 takes 12.29, 12.28 and 13.07 ms, a closed furnace
 // (8 samples) 7.2, 7.3 and 8.6, 100k triangles 23.8, 23.3 and 22.9; with four
 // hero wavelengths the box takes 15.4, 19.8 and 19.9, 100k triangles 27.2, 30.4
-// and 29.4.  With the six waves of pt_kernel large jobs were slower than there.
+// and 29.4.  At six waves, as pt_kernel had, large jobs were slower than there.
 template <int NS, bool RGB>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RGB ? 5 : 4)))
 pt_sample_kernel(SceneView sc, CameraView cam, RenderView rv, float4 *__restrict__ L) {
